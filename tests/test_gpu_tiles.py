@@ -1,0 +1,75 @@
+"""The GEMM shapes for few rows (d32x32, 64x64), for F32 operands as BF16
+terms (x64x64, x128x128) and the rule that picks among them, at the edges of
+their tiles and of k, on an MI355X through the C ABI."""
+import numpy as np
+import pytest
+
+import turboembed_amd as T
+from turboembed_amd import seam as S
+from turboembed_amd.model import to_bf16_bits
+
+pytestmark = pytest.mark.gpu
+
+EDGES = [(1, 96, 64), (31, 32, 8), (32, 33, 72), (65, 100, 192), (129, 257, 100), (300, 384, 1536), (1100, 768, 320)]
+
+
+def _rounded(x, dtype):
+    if dtype == S.TURBO_DTYPE_F16:
+        return x.astype(np.float16).astype(np.float64)
+    if dtype == S.TURBO_DTYPE_BF16:
+        return (to_bf16_bits(x).astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+    return x.astype(np.float64)
+
+
+def _operands(m, n, k):
+    g = np.random.Generator(np.random.PCG64(m + 3 * n + 7 * k))
+    return (g.standard_normal((m, k)).astype(np.float32), g.standard_normal((n, k)).astype(np.float32),
+            g.standard_normal(n).astype(np.float32))
+
+
+@pytest.mark.parametrize("dtype", [S.TURBO_DTYPE_F32, S.TURBO_DTYPE_F16, S.TURBO_DTYPE_BF16])
+@pytest.mark.parametrize("tile", [0, 20, 21, 22, 23])
+@pytest.mark.parametrize("mnk", EDGES)
+def test_small_and_split_shapes_match_numpy(runtime, dtype, tile, mnk):
+    m, n, k = mnk
+    if dtype != S.TURBO_DTYPE_F32 and k % 8:
+        k += 4   # 16-bit operands come in whole 16-byte vectors
+    a, w, b = _operands(m, n, k)
+    got = T.gemm_check(a, w, b, dtype=dtype, tile=tile)
+    want = _rounded(a, dtype) @ _rounded(w, dtype).T + b
+    # An F32 sum of k products of unit variance: k roundings of at most
+    # 2^-24 of a partial sum (at most about 5 sqrt(k)) if every one went
+    # the same way; they do not, and a tenth of that bounds them.
+    bound = max(0.1 * k * 5 * np.sqrt(k) * 2.0 ** -24, 4e-6)
+    assert np.abs(got - want).max() <= bound, (np.abs(got - want).max(), bound)
+
+
+@pytest.mark.parametrize("mnk", [(200, 300, 772), (300, 256, 3072)])
+def test_bf16_terms_are_no_further_off_than_the_f32_products(runtime, mnk):
+    # Against 64 bits: three BF16 terms an operand, six products, must not
+    # lose to the F32 matrix core's own sums (measured 3.2e-7 against 9.2e-7
+    # at k = 3072).
+    a, w, b = _operands(*mnk)
+    want = a.astype(np.float64) @ w.astype(np.float64).T + b
+    off = [np.linalg.norm(T.gemm_check(a, w, b, tile=t) - want) for t in (1, 20, 22, 23)]
+    assert max(off[1:]) <= off[0], off
+
+
+def test_operands_of_every_magnitude_keep_their_terms(runtime):
+    # Rows and columns scaled by 2^-60 to 2^60: each output's error stays
+    # relative to its own operands.
+    m, n, k = 70, 90, 256
+    a, w, _ = _operands(m, n, k)
+    sa, sw = 2.0 ** np.linspace(-60, 60, m).round(), 2.0 ** np.linspace(60, -60, n).round()
+    for t in (20, 22, 23):
+        got = T.gemm_check((a * sa[:, None]).astype(np.float32), (w * sw[:, None]).astype(np.float32), tile=t)
+        want = a.astype(np.float64) @ w.astype(np.float64).T
+        assert np.abs(got.astype(np.float64) / sa[:, None] / sw[None, :] - want).max() <= 1e-5 * np.sqrt(k)
+
+
+@pytest.mark.parametrize("mnk", [(1, 64, 128), (65, 192, 384), (300, 2304, 768)])
+def test_int8_shapes_have_the_same_bits(runtime, mnk):
+    a, w, b = _operands(*mnk)
+    want = T.gemm_check(a, w, b, dtype=S.TURBO_DTYPE_I8, tile=7)
+    for t in (0, 5, 21):
+        np.testing.assert_array_equal(T.gemm_check(a, w, b, dtype=S.TURBO_DTYPE_I8, tile=t), want)

@@ -16,8 +16,8 @@ OUT = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libturbo_rocm.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
-SOURCES = ["rowwise.hip", "gemm.hip", "attention.hip", "session.cpp", "backend.cpp", "checks.cpp", "rerank.cpp",
-           "autotune.cpp", "allocs.cpp"]
+SOURCES = ["rowwise.hip", "gemm.hip", "gemm_direct.hip", "gemm_f32.hip", "attention.hip", "session.cpp",
+           "backend.cpp", "checks.cpp", "rerank.cpp", "autotune.cpp", "allocs.cpp"]
 
 # The backend's own heap allocations are counted (allocs.cpp): its objects'
 # calls of these go to the __wrap_ functions there first.

@@ -20,6 +20,7 @@
 // blocks are renumbered so that each XCD takes a contiguous run of output
 // tiles, along N first: the run shares its A rows, which then stay in that
 // XCD's L2.
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 #include <cstring>
@@ -29,156 +30,10 @@
 #include "launch.h"
 #include "devmath.h"
 #include "rowmath.h"
+#include "gemm_tile.h"
+#include "gemm_more.h"
 
 namespace rocm {
-
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-
-template <typename T> struct Mma;
-
-typedef int int32x4 __attribute__((ext_vector_type(4)));
-typedef int int32x16 __attribute__((ext_vector_type(16)));
-
-template <> struct Mma<_Float16> {
-    static constexpr int EPM = 8;   // elements a lane feeds one MFMA
-    typedef half8 frag;
-    typedef floatx16 acc;
-    static __device__ __forceinline__ floatx16 run(frag a, frag b, floatx16 c) {
-        return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-    }
-};
-
-template <> struct Mma<__bf16> {
-    static constexpr int EPM = 8;
-    typedef bf16x8 frag;
-    typedef floatx16 acc;
-    static __device__ __forceinline__ floatx16 run(frag a, frag b, floatx16 c) {
-        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-    }
-};
-
-template <> struct Mma<int8_t> {
-    static constexpr int EPM = 16;
-    typedef int32x4 frag;
-    typedef int32x16 acc;
-    static __device__ __forceinline__ int32x16 run(frag a, frag b, int32x16 c) {
-        return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
-    }
-};
-
-template <> struct Mma<float> {
-    static constexpr int EPM = 1;
-    typedef float frag;
-    typedef floatx16 acc;
-    static __device__ __forceinline__ floatx16 run(frag a, frag b, floatx16 c) {
-        return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-    }
-};
-
-// A gated unit's product act(gate) * up as stored: at an F16 output it
-// saturates at F16's largest finite magnitude instead of rounding to
-// infinity (a NaN stays NaN), as the reference's CUDA backend stores it
-// (core/cuda/rotary.cuh:31-45); BF16 and F32 outputs hold it as it is.
-template <typename T> __device__ __forceinline__ float gated_product(float g, float up) {
-    const float v = __fmul_rn(g, up);
-    if constexpr (std::is_same<T, _Float16>::value) return v > 65504.0f ? 65504.0f : v < -65504.0f ? -65504.0f : v;
-    return v;
-}
-
-// The rows a GEMM launch multiplies: its span, and how far apart A's token
-// rows are for the span's first token (the run's operand rows may be wider
-// than the product's K).
-struct GemmRows {
-    Span sp;
-    int a_tok;
-};
-
-// The span's first token moves the epilogue's row-major output (and the int8
-// activation scales) down to it; the Q, K and V scatter (and the rotary
-// epilogue's positions) take it as the token of row 0.
-template <Epi KIND, typename OT>
-__device__ __forceinline__ void place_epilogue(EpiArgs &e, const Live &lv) {
-    e.tok0 = lv.tok0;
-    if (e.a_scale) e.a_scale += lv.tok0;
-    const size_t rows = (size_t)lv.tok0 * e.ldo;
-    if constexpr (KIND == Epi::Plain) e.out = (float *)e.out + rows;
-    else if constexpr (KIND == Epi::Bias) e.out = e.out_f32 ? (void *)((float *)e.out + rows) : (void *)((OT *)e.out + rows);
-    else if constexpr (KIND == Epi::Gelu || KIND == Epi::Gated) e.out = (OT *)e.out + rows;
-    else if constexpr (KIND == Epi::Residual) e.x += rows;
-}
-
-// The epilogue of one 32 x 32 MFMA tile, for this lane's column n and its 16
-// rows m0 + 8 (r / 4) + 4 (lane / 32) + r % 4, v = acc + bias. The kind is a
-// template argument, so each kernel carries one small epilogue, and what
-// depends on the column alone is worked out once per tile.
-template <typename T, Epi KIND>
-__device__ __forceinline__ void epilogue_tile(const EpiArgs &e, int M, int N, int mt, int n, const floatx16 &acc) {
-    const int lane = threadIdx.x & 63;
-    const int mb = mt + (lane >> 5) * 4;   // row of register r: mb + 8 (r / 4) + r % 4
-    const bool col_ok = n < N;
-    const float bias = (e.bias && col_ok) ? e.bias[n] : 0.0f;
-    if constexpr (KIND == Epi::Plain || KIND == Epi::Gelu || KIND == Epi::Residual || KIND == Epi::Bias) {
-        if (!col_ok) return;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int m = mb + (r >> 2) * 8 + (r & 3);
-            if (m >= M) continue;
-            const float v = acc[r] + bias;
-            const size_t at = (size_t)m * e.ldo + n;
-            if constexpr (KIND == Epi::Plain) ((float *)e.out)[at] = v;
-            else if constexpr (KIND == Epi::Bias) {
-                if (e.out_f32) ((float *)e.out)[at] = v;
-                else if (sizeof(T) == 2 && e.out_bf16) ((__bf16 *)e.out)[at] = from_f32<__bf16>(v);
-                else ((T *)e.out)[at] = from_f32<T>(v);
-            }
-            else if constexpr (KIND == Epi::Gelu)
-                ((T *)e.out)[at] = from_f32<T>(sizeof(T) == 2 ? dev_gelu_fast(v) : dev_gelu(v));
-            else e.x[at] = e.x[at] + v;
-        }
-    } else if constexpr (KIND == Epi::Qkv || KIND == Epi::QkvRope) {
-        const int which = n / e.hidden, rem = n - which * e.hidden;
-        const int head = rem / e.d, c = rem - head * e.d;
-        T *out = (T *)e.out + (size_t)which * e.heads * e.tcap * e.d;
-        const int half = e.d >> 1, pr = c >> 1;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int m = mb + (r >> 2) * 8 + (r & 3);
-            float v = acc[r] + bias;
-            if constexpr (KIND == Epi::QkvRope) {
-                // Columns come pair-adjacent: the partner of n is n ^ 1, in
-                // the neighbouring lane (column n sits in lane n % 32).
-                const float w = __shfl_xor(v, 1, 64);
-                if (which < 2 && col_ok && m < M) {
-                    // Rounded products, then their sum or difference, in
-                    // every instantiation (no fused multiply-add).
-#pragma clang fp contract(off)
-                    const int pos = e.pos[e.tok0 + m];
-                    const float cs = e.cos[(size_t)pos * half + pr], sn = e.sin[(size_t)pos * half + pr];
-                    // (x1, x2) -> (x1 cos - x2 sin, x2 cos + x1 sin)
-                    v = (c & 1) ? v * cs + w * sn : v * cs - w * sn;
-                }
-            }
-            if (!col_ok || m >= M) continue;
-            // Q and K token-major per head; V transposed per head.
-            const size_t t = (size_t)e.tok0 + m;
-            const size_t at = which < 2 ? ((size_t)head * e.tcap + t) * e.d + c : ((size_t)head * e.d + c) * e.tcap + t;
-            out[at] = from_f32<T>(v);
-        }
-    } else {   // Gated: out[m, n / 2] = act(gate) * up, gate and up in neighbouring columns
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int m = mb + (r >> 2) * 8 + (r & 3);
-            const float v = acc[r] + bias;
-            const float up = __shfl_xor(v, 1, 64);
-            if (!col_ok || m >= M || (n & 1)) continue;
-            const float g = e.silu ? dev_silu(v) : sizeof(T) == 2 ? dev_gelu_fast(v) : dev_gelu(v);
-            ((T *)e.out)[(size_t)m * e.ldo + (n >> 1)] = from_f32<T>(gated_product<T>(g, up));
-        }
-    }
-}
 
 // ks > 0: split K, the grid's y-th slice of ks columns of k (W's rows stay
 // K long), its F32 sums (Plain epilogue, no bias) into slice y of the
@@ -1375,7 +1230,7 @@ hipError_t gemm_ln(hipStream_t s, Dt dt, const Span &sp, int max_m, int hidden, 
 }
 
 // The highest block-shape number.
-constexpr int TILES = 19;
+constexpr int TILES = 23;
 
 int gemm_tiles() { return TILES; }
 
@@ -1400,11 +1255,13 @@ bool gemm_made_to_fail(int tile) {
 
 // Names of the block shapes, as a choices string spells them: output tile,
 // then what sets it apart (r: operands staged through registers; k32: 32
-// columns of k a stage; s<n>: n stages).
+// columns of k a stage; s<n>: n stages; d: K shared among the workgroup's
+// waves, operands straight into registers; x: F32 operands as BF16 terms).
 static const char *const TILE_NAME[TILES + 1] = {
     "auto",      "r128x128",   "r256x128",     "r64x128",    "256x128", "128x128", "128x256",
     "256x256",   "128x128s2",  "256x128k32",   "128x256k32", "256x128k32s3", "256x256k32", "256x192",
-    "r64x64",    "256x384",    "256x384k32s4", "128x768ln", "r128x128sk4", "r64x64sk2"};
+    "r64x64",    "256x384",    "256x384k32s4", "128x768ln", "r128x128sk4", "r64x64sk2",
+    "d32x32",    "64x64",      "x64x64",      "x128x128"};
 
 const char *gemm_tile_name(int tile) { return tile >= 0 && tile <= TILES ? TILE_NAME[tile] : "?"; }
 
@@ -1431,6 +1288,7 @@ static int wave_cols(int tile) {
     case 15:
     case 16: return 96;
     case 4: case 5: case 7: case 8: case 9: case 11: case 12: return 64;
+    case 21: return 32;
     default: return 1;
     }
 }
@@ -1449,6 +1307,8 @@ int gemm_candidates(Dt dt, int K, int lda, const EpiArgs &e, int *out, int cap) 
         if (K % 128 == 0) add(7);
         // (Not with the rotary epilogue, whose angles spill this shape's registers.)
         if (K % 128 == 0 && fits(15) && e.kind != Epi::QkvRope) add(15);
+        if (K % 128 == 0) add(5);
+        if (K % 128 == 0 && fits(21)) add(21);
         add(9);
         return n;
     }
@@ -1457,9 +1317,12 @@ int gemm_candidates(Dt dt, int K, int lda, const EpiArgs &e, int *out, int cap) 
         add(2);
         add(3);
         add(14);
+        add(20);
+        if (dt == Dt::F32) add(22);
+        if (dt == Dt::F32) add(23);
         return n;
     }
-    for (int t : {7, 13, 15, 16, 4, 6, 5, 9, 10})
+    for (int t : {7, 13, 15, 16, 4, 6, 5, 9, 10, 21, 20})
         if (fits(t)) add(t);
     return n;
 }
@@ -1477,36 +1340,94 @@ static int cu_count() {
     return n;
 }
 
-// The pipelined block shape for a large product: 256 x 256 output tiles,
-// or 256 x 192 on a long inner dimension when they leave the compute units
-// less idle over the launch's rounds of tiles (time ~ rounds x tile area).
-// Measured on MI355X at 32768 tokens: 256 x 192 is faster at N = 768,
-// K = 3072 (whole rounds against one and a half), slower at K = 768, where
-// its 96-column waves' operand reads and epilogue cost more than the rounds
-// save. Q, K and V must each start on a wave's column boundary (64 or 96).
-static int wide_tile(int M, int N, int K, const EpiArgs &e) {
+// Rounds of bm x bn output tiles an M x N product takes, `at_once` workgroups
+// running together.
+static double rounds(int M, int N, int bm, int bn, long at_once) {
+    const long tiles = (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+    return (double)((tiles + at_once - 1) / at_once);
+}
+
+// The rule's block shape for a product of at most M rows. A launch takes
+// about its rounds of tiles over the compute units times its shape's time a
+// round, which a small tile spends mostly waiting (K / 64 stages behind a
+// barrier each), so small tiles win while they fit in few rounds and large
+// ones, with fewer operand reads a product, once the chip is full. Times a
+// round relative to 64 x 64 tiles, measured on MI355X at K = 768 (5.8 us;
+// within 10% of the same ratios at 384 and 3072): 128 x 128 2.1, 256 x 192
+// 3.7, 256 x 256 4.3. So at N = 768 (us): 256 rows 6.0 on 64 x 64 against
+// 10.9 on 128 x 128; 4096 rows 14.1 on 128 x 128 against 16.5 on 64 x 64
+// and 25.4 on 256 x 256; at N = 2304, 1024 rows 14.8 on 128 x 128 against
+// 17.5 and 26.2, 4096 rows 27.3 on 256 x 192 against 42 on 128 x 128 and
+// 31 on 256 x 256.
+// Past one round, 256 x 192 is for long inner dimensions: measured at 32768
+// rows it is faster at N = 768, K = 3072 (whole rounds against one and a
+// half), slower at K = 768, where its 96-column waves' operand reads and
+// epilogue cost more than the rounds save. Q, K and V must each start on a
+// wave's column boundary (32, 64 or 96).
+static int pipelined_tile(int M, int N, int K, const EpiArgs &e) {
     const bool qkv = e.kind == Epi::Qkv || e.kind == Epi::QkvRope;
     const long cus = cu_count();
-    auto cost = [&](int bm, int bn) {
-        const long tiles = (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-        return (double)((tiles + cus - 1) / cus) * bm * bn;
+    const double wide = 4.3 * rounds(M, N, 256, 256, cus), r192 = rounds(M, N, 256, 192, cus);
+    int tile = 7;
+    double best = wide;
+    auto take = [&](int t, double cost) {
+        if (cost < best && !gemm_made_to_fail(t)) {
+            best = cost;
+            tile = t;
+        }
     };
-    const bool can192 = (!qkv || e.hidden % 96 == 0) && K >= 2048;
-    if (can192 && cost(256, 192) * 1.03 < cost(256, 256)) return 13;
-    return 7;
+    // (One round of 32 x 32 tiles: 768 x 3072 at 24 rows 12 us against 13.)
+    if (rounds(M, N, 32, 32, cus) <= 1 && !gemm_made_to_fail(20)) return 20;
+    if ((!qkv || e.hidden % 96 == 0) && (K >= 2048 || r192 <= 1)) take(13, 3.7 * 1.03 * r192);
+    take(5, 2.1 * rounds(M, N, 128, 128, cus));
+    take(21, 1.0 * rounds(M, N, 64, 64, cus));
+    return tile;
+}
+
+int gemm_split_tile(Dt dt, int M, int N, int K, int parts, const EpiArgs &e) {
+    const double at_once = std::max(1, cu_count() / parts);
+    auto cost = [&](double round, int bm, int bn) {
+        const double tiles = (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+        return round * std::max(1.0, tiles / at_once);
+    };
+    int cand[16];
+    const int n = gemm_candidates(dt, K, K, e, cand, 16);
+    auto can = [&](int t) { return std::find(cand, cand + n, t) != cand + n && !gemm_made_to_fail(t); };
+    if (!can(WIDE_TILE)) return 0;
+    return dt != Dt::I8 && can(13) && cost(3.7, 256, 192) < 0.9 * cost(5.9, 256, 384) ? 13 : WIDE_TILE;
+}
+
+// The rule for operands the pipelined kernel does not take (F32, or K not a
+// multiple of 64). Few rows: 32 x 32 tiles with K shared among a
+// workgroup's waves (gemm_direct.hip), while at most three workgroups a CU
+// (F32 384 x 1536 at 1024 rows 37 us against 38 on 64 x 64 tiles of BF16
+// terms; 768 x 3072 at 512 rows 68 against 88, at 1024 rows 104 against 86).
+// Then F32 takes its BF16 terms (gemm_f32.hip) on 64 x 64 tiles, two
+// workgroups a CU at about 30 us a round at K = 768, or on 128 x 128 ones
+// at 44 (2300 rows: N = 768 31 us against 44, N = 1536, K = 384 40 against 32).
+static int staged_tile(Dt dt, int M, int N) {
+    const long cus = cu_count();
+    if (!gemm_made_to_fail(20) && (M <= 256 || rounds(M, N, 32, 32, 3 * cus) <= 1)) return 20;
+    if (dt != Dt::F32) return 1;
+    return 30 * rounds(M, N, 64, 64, 2 * cus) <= 44 * rounds(M, N, 128, 128, cus) ? 22 : 23;
 }
 
 // Block shapes by number: 1-3 and 14 stage operands through registers (any K
-// a multiple of 8, and the F32 tier); 4-13, 15 and 16 are the pipelined
-// kernel, for 16-bit operands with K a multiple of 64 (every encoder shape
+// a multiple of 8, and the F32 tier); 20 shares K among its waves (the same
+// operands); 22 and 23 take F32 operands as BF16 terms; 4-13, 15, 16 and 21
+// are the pipelined kernel, for 16-bit operands with K a multiple of 64 (every encoder shape
 // here).
+template <typename T> constexpr Dt dt_of() {
+    return sizeof(T) == 4 ? Dt::F32 : std::is_same<T, __bf16>::value ? Dt::BF16 : Dt::F16;
+}
+
 template <typename T, int BK>
 static hipError_t gemm_t(hipStream_t s, const GemmRows &gr, int M, int N, int K, const void *A, int lda, const void *W,
                          const EpiArgs &e,
                          int tile) {
     const bool pipelined = sizeof(T) == 2 && K % 64 == 0 && lda % 8 == 0;
     if (tile == 0) {
-        tile = pipelined ? (M >= 2048 ? wide_tile(M, N, K, e) : 5) : 1;
+        tile = pipelined ? pipelined_tile(M, N, K, e) : staged_tile(dt_of<T>(), M, N);
         // The rule's next choices when its own cannot launch here.
         static const int PIPELINED[] = {7, 4, 5, 6, 8}, STAGED[] = {1, 2, 3, 14, 0};
         const int *next = pipelined ? PIPELINED : STAGED;
@@ -1514,11 +1435,12 @@ static hipError_t gemm_t(hipStream_t s, const GemmRows &gr, int M, int N, int K,
     }
     if (gemm_made_to_fail(tile)) return hipErrorInvalidDeviceFunction;
     // A pipelined shape asked of an operand it cannot take runs the staged kernel.
-    if (((tile >= 4 && tile <= 13) || tile == 15 || tile == 16) && !pipelined) tile = (N % 128 == 0 && M >= 8192) ? 2 : 1;
+    if (((tile >= 4 && tile <= 13) || tile == 15 || tile == 16 || tile == 21) && !pipelined) tile = (N % 128 == 0 && M >= 8192) ? 2 : 1;
     // Q, K and V must each start on a wave's column boundary: a shape whose
     // waves are wider than 64 columns runs 64-column waves (K = hidden is a
     // multiple of 64 on the pipelined kernel) when they do not.
     if ((e.kind == Epi::Qkv || e.kind == Epi::QkvRope) && e.hidden % wave_cols(tile) != 0) tile = 7;
+    if (sizeof(T) == 2 && (tile == 22 || tile == 23)) tile = pipelined ? 5 : 1;   // (F32 operands alone)
     switch (tile) {
     // Split K: the staged kernel's tiles over K in 4 (128 x 128) or 2 (64 x 64) slices.
     case SPLITK_TILE_4: return launch_split<T, 128, 128, BK>(s, gr, M, N, K, A, lda, W, e, 4);
@@ -1528,6 +1450,11 @@ static hipError_t gemm_t(hipStream_t s, const GemmRows &gr, int M, int N, int K,
     case 3: return launch<T, 64, 128, BK>(s, gr, M, N, K, A, lda, W, e);
     // 64 x 64: four times the workgroups of 128 x 128, for products too small to fill the chip.
     case 14: return launch<T, 64, 64, BK>(s, gr, M, N, K, A, lda, W, e);
+    // 32 x 32, K shared among the workgroup's waves: a few rows.
+    case 20: return gemm_direct(s, dt_of<T>(), gr, M, N, K, A, lda, W, e);
+    }
+    if constexpr (sizeof(T) == 4) {
+        if (tile == 22 || tile == 23) return gemm_f32_split(s, tile == 23, gr, M, N, K, A, lda, W, e);
     }
     if constexpr (sizeof(T) == 2) {
         switch (tile) {
@@ -1549,26 +1476,38 @@ static hipError_t gemm_t(hipStream_t s, const GemmRows &gr, int M, int N, int K,
         // The same waves on 32 columns of k a stage, four stages (all 160 KB
         // of LDS): loads issued three steps ahead instead of one.
         case 16: return launch_lds<T, 256, 384, 2, 4, 4, 32, 1>(s, gr, M, N, K, A, lda, W, e);
+        case 21: return launch_lds<T, 64, 64, 2, 2, 4>(s, gr, M, N, K, A, lda, W, e);
         }
     }
     return hipErrorInvalidValue;
 }
 
+// The rule's block shape on 128-byte int8 rows: as pipelined_tile, every shape
+// having the same bits.
+static int i8_tile(int M, int N) {
+    const long cus = cu_count();
+    const double wide = 4.3 * rounds(M, N, 256, 256, cus), mid = 2.1 * rounds(M, N, 128, 128, cus),
+                 small = rounds(M, N, 64, 64, cus);
+    return small < mid && small < wide ? 21 : mid < wide ? 5 : 7;
+}
+
 // The int8 tier: the pipelined kernel alone, on 128-byte rows (K a multiple
-// of 128: 256 x 256 or 256 x 384 tiles) or 64-byte rows (K a multiple of 64).
+// of 128: 64 x 64, 128 x 128, 256 x 256 or 256 x 384 tiles) or 64-byte rows (K a multiple of 64).
 static hipError_t gemm_i8(hipStream_t s, const GemmRows &gr, int M, int N, int K, const void *A, int lda, const void *W,
                           const EpiArgs &e,
                           int tile) {
     if (K % 64 != 0 || lda % 16 != 0 || !e.a_scale || !e.w_scale) return hipErrorInvalidValue;
     if (tile == 0) {
-        tile = K % 128 == 0 ? 7 : 9;
+        tile = K % 128 == 0 ? i8_tile(M, N) : 9;
         if (gemm_made_to_fail(tile)) tile = tile == 7 ? 9 : 7;
     }
-    if ((tile == 7 || tile == 15) && K % 128 != 0) tile = 9;
+    if (tile != 9 && K % 128 != 0) tile = 9;
     if (gemm_made_to_fail(tile)) return hipErrorInvalidDeviceFunction;
     switch (tile) {
     case 7: return launch_lds<int8_t, 256, 256, 2, 4, 2, 128, 1>(s, gr, M, N, K, A, lda, W, e);
     case 15: return launch_lds<int8_t, 256, 384, 2, 4, 2, 128, 1>(s, gr, M, N, K, A, lda, W, e);
+    case 5: return launch_lds<int8_t, 128, 128, 2, 2, 4, 128, 1>(s, gr, M, N, K, A, lda, W, e);
+    case 21: return launch_lds<int8_t, 64, 64, 2, 2, 4, 128, 1>(s, gr, M, N, K, A, lda, W, e);
     default: return launch_lds<int8_t, 256, 128, 2, 2, 2, 64, 2>(s, gr, M, N, K, A, lda, W, e);
     }
 }

@@ -189,6 +189,9 @@ int gemm_tile_by_name(const char *s, size_t n);
 int gemm_candidates(Dt dt, int K, int lda, const EpiArgs &e, int *out, int cap);
 // The 256 x 384 block shape (8 waves of 128 x 96): a split run's products' shape.
 constexpr int WIDE_TILE = 15;
+// The block shape for a product that runs beside those of the run's other
+// parts, of at most M rows a part (0: the launcher's rule).
+int gemm_split_tile(Dt dt, int M, int N, int K, int parts, const EpiArgs &e);
 // A post-norm product of N = hidden with the residual add and the LayerNorm
 // in its epilogue (whole-row tiles): y = A W^T + bias rounded to the operand
 // type, v = out_h + y, out_h = LN(v) (and x = LN(v) in F32 with keep_f32),

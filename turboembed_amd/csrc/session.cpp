@@ -758,6 +758,12 @@ Session *session_open(Model *m, const turbo_backend_session_desc *desc, turbo_ba
     s->pool_scratch.chunks = (int)((S + POOL_CHUNK - 1) / POOL_CHUNK);
     s->pool_scratch.part = static_cast<float *>(alloc(outs * s->pool_scratch.chunks * H * 4, "session pooling"));
     s->pool_scratch.cnt = static_cast<int32_t *>(alloc(outs * s->pool_scratch.chunks * 4, "session pooling"));
+    if (s->task == TURBO_TASK_RERANK) {
+        s->head_w = static_cast<float *>(alloc((H * H + 2 * H) * 4, "session rerank head"));
+        s->pooled = static_cast<float *>(alloc(B * H * 4, "session rerank head"));
+        s->logits = static_cast<float *>(alloc(2 * B * 4, "session rerank head"));
+        s->finite = reinterpret_cast<int32_t *>(s->logits + B);
+    }
     s->output.ctx = m->ctx;
     s->output.placement = TURBO_PLACE_DEVICE;
     s->output.dev = s->out;
@@ -833,29 +839,55 @@ static uint32_t parts_of_bin(const Session &s, int b) {
     return splits && s.split_parts > 1 && s.max_batch >= 2 ? std::min(s.split_parts, s.max_batch) : 1;
 }
 
+// How large a run's launches are: every grid covers the largest run of the
+// bin (whose kernel choices they take), so the launches of a bin are the same
+// whether captured into its graph or launched directly, and give the same
+// bits. A part's tokens are at most a share of the bin's plus one row (its
+// last row crosses the share) plus one (the share's rounding).
+struct Bounds {
+    int bin = 0;
+    uint32_t tokens = 0, rows = 0, max_len = 0, parts = 1, part_tokens = 0, items = 0;
+};
+
+static Bounds bounds_of(const Session &s, int b, uint32_t parts) {
+    Bounds o;
+    o.bin = b;
+    o.tokens = bin_tokens(b, (uint64_t)s.max_batch * s.max_seq);
+    o.rows = std::min<uint32_t>(s.max_batch, o.tokens);
+    o.max_len = std::min<uint32_t>(s.max_seq, o.tokens);
+    o.parts = std::max(parts, 1u);
+    const uint32_t bp = o.parts;
+    o.part_tokens = bp == 1 ? o.tokens : std::min(o.tokens, (o.tokens + bp - 1) / bp + 1 + o.max_len);
+    o.items = std::max(o.rows, s.max_ranges);
+    return o;
+}
+
 // The rule's choice in a bin whose runs split into parts: the 256 x 384
-// block shape on every product that can take it. The parts run the same
-// kernels side by side, and shapes fastest alone lose there: a 256 x 384
-// product at N = 768 fills half the compute units and the other part's the
-// rest. Measured on MI355X, a batch with it on all four products against
-// the shapes the tuner finds fastest alone: BERT-base 64 x 512 8.05 ms
-// against 8.23-8.35, ModernBERT 16 x 2048-8192 45.4-45.6 ms against
-// 45.4-46.6 (timing whole runs in the tuner could not tell them apart
-// reliably: its short bursts run at clocks a sustained run does not).
+// block shape on every product that can take it, or 256 x 192 where the
+// parts' tiles leave compute units idle. The parts run the same kernels side
+// by side, and shapes fastest alone lose there: a 256 x 384 product at N =
+// 768 fills half the compute units and the other part's the rest. Measured
+// on MI355X, a batch with it on all four products against the shapes the
+// tuner finds fastest alone: BERT-base 64 x 512 8.05 ms against 8.23-8.35,
+// ModernBERT 16 x 2048-8192 45.4-45.6 ms against 45.4-46.6 (timing whole
+// runs in the tuner could not tell them apart reliably: its short bursts run
+// at clocks a sustained run does not). In the le16k bin, and at hidden 384,
+// its residual products' tiles are too few (16,384 tokens: 128 at N = 768).
 static void split_defaults(Session &s) {
     const Model &m = *s.model;
     for (int b = 0; b < s.kc.bins; ++b) {
-        if (parts_of_bin(s, b) < 2) continue;
+        const uint32_t parts = parts_of_bin(s, b);
+        if (parts < 2) continue;
         BinChoice &bc = s.kc.bin[b];
+        const Bounds bd = bounds_of(s, b, parts);
         for (int g = 0; g < G_COUNT; ++g) {
-            if (bc.tile_forced[g] || gemm_made_to_fail(WIDE_TILE)) continue;
+            if (bc.tile_forced[g]) continue;
             EpiArgs e;
             e.kind = g == G_QKV ? Epi::Qkv : Epi::Bias;
             e.hidden = (int)m.hidden;
             const int K = g == G_FFN2 ? (int)m.inter : (int)m.hidden;
-            int cand[16];
-            const int n = gemm_candidates(s.dt, K, K, e, cand, 16);
-            if (std::find(cand, cand + n, WIDE_TILE) != cand + n) bc.tile[g] = WIDE_TILE;
+            const int N = (int)(g == G_QKV ? m.ls[0].n_qkv : g == G_FFN1 ? m.ls[0].n_in : m.hidden);
+            if (const int t = gemm_split_tile(s.dt, (int)bd.part_tokens, N, K, (int)parts, e)) bc.tile[g] = t;
         }
     }
 }
@@ -1151,29 +1183,6 @@ static LayerGemm layer_gemm(Session &s, uint32_t l, GemmSlot g) {
         break;
     }
     return r;
-}
-
-// How large a run's launches are: every grid covers the largest run of the
-// bin (whose kernel choices they take), so the launches of a bin are the same
-// whether captured into its graph or launched directly, and give the same
-// bits. A part's tokens are at most a share of the bin's plus one row (its
-// last row crosses the share) plus one (the share's rounding).
-struct Bounds {
-    int bin = 0;
-    uint32_t tokens = 0, rows = 0, max_len = 0, parts = 1, part_tokens = 0, items = 0;
-};
-
-static Bounds bounds_of(const Session &s, int b, uint32_t parts) {
-    Bounds o;
-    o.bin = b;
-    o.tokens = bin_tokens(b, s.tcap);
-    o.rows = std::min<uint32_t>(s.max_batch, o.tokens);
-    o.max_len = std::min<uint32_t>(s.max_seq, o.tokens);
-    o.parts = std::max(parts, 1u);
-    const uint32_t bp = o.parts;
-    o.part_tokens = bp == 1 ? o.tokens : std::min(o.tokens, (o.tokens + bp - 1) / bp + 1 + o.max_len);
-    o.items = std::max(o.rows, s.max_ranges);
-    return o;
 }
 
 // Post-norm F16 sessions carry the residual stream between a layer's norms
