@@ -1,0 +1,49 @@
+"""Attention with F32 probabilities on the matrix cores (F32 heads of 32 and
+64, 16-bit heads of 32): rows at the edges of its 32-query, 32-key and
+128-query blocks, masked keys through them, and windows, against the oracle on
+an MI355X through the C ABI."""
+import numpy as np
+import pytest
+
+import oracle
+from turboembed_amd import seam as S
+from turboembed_amd.model import with_dtype
+
+import small
+from test_gpu_parity import assert_close
+
+pytestmark = pytest.mark.gpu
+
+
+# (Heads of 64 on the F32 tier alone: the 16-bit ones take the other kernel.)
+@pytest.mark.parametrize("tier, heads", [("f32", 4), ("f32", 2), ("f16", 4), ("bf16", 4)])
+@pytest.mark.parametrize("family, window", [("bert", 0), ("modernbert", 16), ("modernbert", 40)])
+def test_rows_at_block_edges_meet_the_oracle(context, tier, heads, family, window):
+    # Weights N(0, 0.3) spread the scores over tens of units; N(0, 0.1) on
+    # BF16, whose operands' rounding (2^-9 of each, the scores' 2^-9 of tens)
+    # alone moves such softmaxes past the dtype's floor, as it does on the
+    # kernel for heads of 64.
+    seq, std = 300, 0.1 if tier == "bf16" else 0.3
+    if family == "bert":
+        desc = small.bert(seed=51, hidden=128, heads=heads, inter=256, positions=seq, std=std)
+    else:
+        desc = small.modernbert(seed=51, hidden=128, heads=heads, inter=192, positions=seq, window=window,
+                                global_every=2, std=std)
+    precision = S.TURBO_PRECISION_EXACT if tier == "f32" else S.TURBO_PRECISION_FASTEST
+    if tier == "bf16":
+        desc, precision = with_dtype(desc, "bf16"), S.TURBO_PRECISION_MODEL
+    g = np.random.Generator(np.random.PCG64(51))
+    lens = [1, 2, 31, 32, 33, 63, 64, 65, 127, 128, 129, 257, 300]
+    ids = g.integers(0, desc.vocab_size, size=(len(lens), seq)).astype(np.int32)
+    mask = (np.arange(seq)[None, :] < np.array(lens)[:, None]).astype(np.int32)
+    mask[8, 32:64] = 0             # a whole block of masked keys
+    mask[10, [0, 31, 32, 96]] = 0
+    mask[12, 5:290:3] = 0
+    types = g.integers(0, 2, size=ids.shape).astype(np.int32) if family == "bert" else None
+    model = context.load(desc)
+    s = model.session(len(lens), seq, precision)
+    got = s.embed(ids, mask, types)
+    assert_close(got, oracle.encode(desc, ids, mask, types), s.compute_dtype)
+    assert np.array_equal(s.embed(ids, mask, types), got)
+    s.close()
+    model.close()

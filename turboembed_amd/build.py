@@ -16,8 +16,9 @@ OUT = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libturbo_rocm.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
-SOURCES = ["rowwise.hip", "gemm.hip", "gemm_direct.hip", "gemm_f32.hip", "attention.hip", "session.cpp",
-           "backend.cpp", "checks.cpp", "rerank.cpp", "autotune.cpp", "allocs.cpp"]
+SOURCES = ["rowwise.hip", "gemm.hip", "gemm_direct.hip", "gemm_f32.hip", "attention.hip",
+           "attention_f32p.hip", "session.cpp", "backend.cpp", "checks.cpp", "rerank.cpp",
+           "autotune.cpp", "allocs.cpp"]
 
 # The backend's own heap allocations are counted (allocs.cpp): its objects'
 # calls of these go to the __wrap_ functions there first.
@@ -28,7 +29,7 @@ WRAPPED = ["malloc", "calloc", "realloc", "aligned_alloc", "posix_memalign", "_Z
 # so the softmax's vector ops on its accumulators need no copies through the
 # accumulation registers; and no NaN operands (its inputs are finite), so a
 # max of scores is one v_max3_f32 without a quieting v_max_f32 per score.
-EXTRA = {"attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-fno-honor-nans"]}
+EXTRA = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form", "-fno-honor-nans"] for f in ("attention.hip", "attention_f32p.hip")}
 
 FLAGS = [
     "-O3", "-std=c++17", "-fPIC", "--offload-arch=gfx950",

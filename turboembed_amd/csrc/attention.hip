@@ -19,7 +19,8 @@ namespace rocm {
 // online softmax in F32 on Cephes' exp (a key's dot product in column order,
 // one FMA chain). The waves' states then merge: each rescales its context and
 // sum to the largest of their maxima, and wave 0 adds the contexts and sums in
-// wave order. Every tier's reference path.
+// wave order. Every 16-bit tier's reference path at heads of 64, and the
+// path of the head widths with no matrix-core one (8, 16 and 128).
 constexpr int SW = 4;
 template <typename T, int D>
 __global__ void __launch_bounds__(64 * SW) attention_simple_kernel(const T *__restrict__ qkv, int tcap, int heads,
@@ -133,9 +134,15 @@ static hipError_t attention_t(hipStream_t s, const void *qkv, int tcap, int head
     switch (d) {
         ATT_CASE(8)
         ATT_CASE(16)
-        ATT_CASE(32)
-        ATT_CASE(64)
         ATT_CASE(128)
+    case 64:
+        // (16-bit operands alone: attention_f32p takes F32's.)
+        if constexpr (sizeof(T) == 2) {
+            enqueue((attention_simple_kernel<T, 64>), grid, dim3(64 * SW), 0, s, (const T *)qkv, tcap, heads, p, mask,
+                    sp, window, (T *)ctx);
+            break;
+        }
+        return hipErrorInvalidValue;
     default: return hipErrorInvalidValue;
     }
 #undef ATT_CASE
@@ -663,6 +670,8 @@ hipError_t attention(hipStream_t s, Dt dt, const void *qkv, int tcap, int heads,
                      int path) {
     if (max_len <= 0 || max_rows <= 0) return hipSuccess;
     if (path < 0 || path > 2) return hipErrorInvalidValue;
+    if (attention_f32p_takes(dt, d))
+        return attention_f32p(s, dt, qkv, tcap, heads, d, p, mask, sp, max_rows, max_len, window, ctx);
     const bool mfma = d == 64 && path != 1;
     switch (dt) {
     case Dt::F16:

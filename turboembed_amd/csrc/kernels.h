@@ -232,14 +232,22 @@ bool gemm_made_to_fail(int tile);
 // qkv, into ctx [tokens, heads * d] in `dt`. window: keys within `window` of
 // the query (|i - j| <= window), or INT32_MAX. F16 and BF16 heads of 64 run
 // on the matrix cores (path 0: 256-query workgroups; 2: 128-query ones)
-// unless path is 1; F32 runs the scalar path.
+// unless path is 1; F32 heads of 32 and 64 and 16-bit heads of 32 run there
+// with F32 probabilities (attention_f32p) whatever the path, and other widths
+// the scalar path.
 // The span's rows; max_rows and max_len bound the grid.
 hipError_t attention(hipStream_t s, Dt dt, const void *qkv, int tcap, int heads, int d, const Packing &p,
                      const int32_t *mask, const Span &sp, int max_rows, int max_len, int window, void *ctx,
                      int path = 0);
 
-// A mean's tokens are summed in chunks of POOL_CHUNK, each chunk in token
-// order by its own workgroup, then the chunks' sums in chunk order: `part`
+// The matrix-core kernel with F32 probabilities, and the operand types and
+// head widths it takes (attention_f32p.hip).
+bool attention_f32p_takes(Dt dt, int d);
+hipError_t attention_f32p(hipStream_t s, Dt dt, const void *qkv, int tcap, int heads, int d, const Packing &p,
+                          const int32_t *mask, const Span &sp, int max_rows, int max_len, int window, void *ctx);
+
+// A long mean's tokens are summed in chunks of POOL_CHUNK, each chunk by its
+// own workgroup, then the chunks' sums in chunk order: `part`
 // holds [count][chunks][output_dim] F32 sums and `cnt` [count][chunks]
 // token counts, chunks >= ceil(seq / POOL_CHUNK).
 constexpr int POOL_CHUNK = 256;
