@@ -17,7 +17,7 @@ LIB = os.path.join(HERE, "libturbo_rocm.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 SOURCES = ["rowwise.hip", "gemm.hip", "gemm_direct.hip", "gemm_f32.hip", "attention.hip",
-           "attention_f32p.hip", "session.cpp", "backend.cpp", "checks.cpp", "rerank.cpp",
+           "attention_f32p.hip", "head.hip", "session.cpp", "backend.cpp", "checks.cpp", "rerank.cpp",
            "autotune.cpp", "allocs.cpp"]
 
 # The backend's own heap allocations are counted (allocs.cpp): its objects'

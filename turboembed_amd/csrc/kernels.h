@@ -267,6 +267,15 @@ hipError_t pool(hipStream_t s, const RunDims *dims, int max_items, const float *
                 const int32_t *mask, const uint32_t *ranges, const PoolScratch &ps, float *out,
                 const float *hw = nullptr, const float *hb = nullptr, int hout = 0);
 
+// The sequence classification head over `rows` states x [rows, hidden]: with
+// pooler_w [hidden, hidden] (pooler_b [hidden] or NULL) tanh of the pooler's
+// rows into pooled [rows, hidden], then cls_w [hidden] and cls_b over them (or,
+// without a pooler, over x): F64 sums, each result rounded to F32, into
+// logit [rows]; finite [rows] is 0 for a state with an infinity or NaN.
+hipError_t rerank_head(hipStream_t s, const float *x, int rows, int hidden, const float *pooler_w,
+                       const float *pooler_b, const float *cls_w, float cls_b, float *pooled, float *logit,
+                       int32_t *finite);
+
 // The MFMA rate probe: `blocks` workgroups of 4 waves, each wave 8 chains of
 // 32x32x16 F16 products for `iters` rounds, fixed or random operands; out
 // takes 256 floats, clk the shader and real-time (100 MHz) counts of one wave.

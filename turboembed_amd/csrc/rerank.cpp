@@ -119,7 +119,8 @@ int32_t turbo_rocm_rerank_run(void *session, const int32_t *ids, const int32_t *
                               float classifier_bias, float *scores, turbo_error *err) {
     return guarded(err, [&] {
         Session *s = static_cast<Session *>(session);
-        if (!s || !ids || !types || !lengths || !owner || !scores || windows == 0 || pairs == 0 || seq == 0)
+        if (!s || !ids || !types || !lengths || !owner || !scores || !classifier_weight || windows == 0 ||
+            pairs == 0 || seq == 0)
             fail(TURBO_E_INVALID_ARGUMENT, "rerank run: NULL arguments or zero counts");
         if (s->task != TURBO_TASK_RERANK) fail(TURBO_E_UNSUPPORTED_TASK, "model task is not rerank");
         if (pairs > s->max_batch) fail(TURBO_E_CAPACITY, "pair count exceeds max_batch");
@@ -130,9 +131,23 @@ int32_t turbo_rocm_rerank_run(void *session, const int32_t *ids, const int32_t *
                 fail(TURBO_E_INVALID_ARGUMENT, "rerank run: window " + std::to_string(w));
         for (uint32_t p = 0; p < pairs; ++p) scores[p] = -std::numeric_limits<float>::infinity();
         std::vector<int32_t> mask((size_t)std::min(windows, s->max_batch) * seq);
-        std::vector<float> states, logits;
-        // Windows in runs of max_batch, each row's CLS state read back and
-        // scored; a pair's score is its best window's.
+        std::vector<float> logits;
+        // The call's head beside the states. (The tensors are the caller's:
+        // copied on every call. A copy from pageable memory has left it when
+        // it returns.)
+        float *const pw = s->head_w, *const pb = pw + (size_t)H * H, *const cw = pb + H;
+        {
+            std::lock_guard<std::recursive_mutex> g(s->ctx->lock);
+            OnDevice on(s->ctx->ordinal);
+            auto upload = [&](float *dst, const float *src, size_t n) {
+                if (src) check(hipMemcpyAsync(dst, src, n * 4, hipMemcpyHostToDevice, s->ctx->stream), "rerank head");
+            };
+            upload(pw, pooler_weight, (size_t)H * H);
+            upload(pb, pooler_bias, H);
+            upload(cw, classifier_weight, H);
+        }
+        // Windows in runs of max_batch, each row's CLS state scored
+        // beside it; a pair's score is its best window's.
         for (uint32_t start = 0; start < windows; start += s->max_batch) {
             const uint32_t n = std::min(windows - start, s->max_batch);
             for (uint32_t r = 0; r < n; ++r)
@@ -154,13 +169,31 @@ int32_t turbo_rocm_rerank_run(void *session, const int32_t *ids, const int32_t *
             run.struct_size = sizeof run;
             rc = turbo_rocm_backend.session_run(session, &run, err);
             if (rc != TURBO_OK) return rc;
-            states.resize((size_t)n * H);
-            rc = turbo_rocm_backend.buffer_read(run.output, states.data(), states.size() * 4, err);
-            if (rc != TURBO_OK) return rc;
             logits.resize(n);
-            rc = turbo_rocm_rerank_scores(states.data(), n, H, pooler_weight, pooler_bias, classifier_weight,
-                                          classifier_bias, logits.data(), err);
-            if (rc != TURBO_OK) return rc;
+            {
+                std::lock_guard<std::recursive_mutex> g(s->ctx->lock);
+                OnDevice on(s->ctx->ordinal);
+                hipStream_t st = s->ctx->stream;
+                check(rerank_head(st, s->out, (int)n, (int)H, pooler_weight ? pw : nullptr,
+                                  pooler_bias ? pb : nullptr, cw, classifier_bias, s->pooled, s->logits, s->finite),
+                      "rerank head");
+                // The logits, then (max_batch on) the finite flags, in one
+                // copy through the context's pinned stage where it has one.
+                const size_t words = (size_t)s->max_batch + n;
+                std::vector<float> pageable;
+                const bool staged = s->ctx->read_stage && words * 4 <= Context::READ_STAGE;
+                if (!staged) pageable.resize(words);
+                float *host = staged ? static_cast<float *>(s->ctx->read_stage) : pageable.data();
+                check(hipMemcpyAsync(host, s->logits, words * 4, hipMemcpyDeviceToHost, st), "rerank head");
+                check(hipStreamSynchronize(st), "rerank head");
+                for (uint32_t r = 0; r < n; ++r) {
+                    int32_t finite;
+                    std::memcpy(&finite, host + s->max_batch + r, 4);
+                    if (!finite) fail(TURBO_E_INTERNAL, "non-finite rerank encoder output");
+                    if (!std::isfinite(host[r])) fail(TURBO_E_INTERNAL, "rerank relevance overflows F32");
+                    logits[r] = host[r];
+                }
+            }
             for (uint32_t r = 0; r < n; ++r) {
                 float &sc = scores[owner[start + r]];
                 sc = std::max(sc, logits[r]);

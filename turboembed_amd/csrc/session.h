@@ -181,6 +181,11 @@ struct Session {
     float *splitk_ws = nullptr;   // split K's F32 slices (not on the int8 tier)
     size_t splitk_floats = 0;
     PoolScratch pool_scratch;   // the means' chunk sums
+    // Rerank sessions: the call's head (pooler [H, H] and its bias [H], the
+    // classifier's row [H]), its pooled rows [max_batch, H], and a logit and
+    // a finite flag a row.
+    float *head_w = nullptr, *pooled = nullptr, *logits = nullptr;
+    int32_t *finite = nullptr;
     Buffer output;
     int32_t *staging = nullptr;   // pinned: ids, mask, types planes then ranges
     size_t staging_ints = 0;
