@@ -418,7 +418,7 @@ add_ln_pair_kernel(Span sp, int hidden, float *__restrict__ x, const Y *__restri
 // Rows a half-wave takes (2: BERT-base 0.9% faster a step than 1, with
 // the weight reads halved; 4 is 2.5% slower, its registers halving the
 // waves a SIMD), and waves a block (4: two-wave blocks were 13% slower).
-constexpr int LN_ROWS = 2, LN_WAVES = 4;
+constexpr int LN_ROWS = 2, LN_WAVES = 4, LN_FEW = 4096;
 
 template <typename H, int G, typename Y>
 static hipError_t add_ln_v(hipStream_t s, const Span &sp, int tokens, int hidden, float *x, const void *y,
@@ -430,9 +430,15 @@ static hipError_t add_ln_v(hipStream_t s, const Span &sp, int tokens, int hidden
     // must give the bits of the fused one.
     if constexpr (sizeof(Y) == 2 && sizeof(H) == 2) {
         if (res_h && hidden % 8 == 0) {
-            enqueue((add_ln_pair_kernel<G, Y, H, true, LN_ROWS, LN_WAVES>),
-                    (pair_blocks<LN_WAVES, LN_ROWS>(tokens)), dim3(64 * LN_WAVES), 0, s,
-                    sp, hidden, x, (const Y *)y, ln_w, ln_b, eps, pre_norm, (int)keep_f32, (H *)out_h, qo);
+            // (Few tokens: a row a half, so no row's sums wait for another's.)
+            if (tokens <= LN_FEW)
+                enqueue((add_ln_pair_kernel<G, Y, H, true, 1, LN_WAVES>), (pair_blocks<LN_WAVES, 1>(tokens)),
+                        dim3(64 * LN_WAVES), 0, s, sp, hidden, x, (const Y *)y, ln_w, ln_b, eps, pre_norm,
+                        (int)keep_f32, (H *)out_h, qo);
+            else
+                enqueue((add_ln_pair_kernel<G, Y, H, true, LN_ROWS, LN_WAVES>),
+                        (pair_blocks<LN_WAVES, LN_ROWS>(tokens)), dim3(64 * LN_WAVES), 0, s,
+                        sp, hidden, x, (const Y *)y, ln_w, ln_b, eps, pre_norm, (int)keep_f32, (H *)out_h, qo);
             return hipGetLastError();
         }
     }
@@ -680,72 +686,88 @@ __device__ __forceinline__ PoolRun pool_run(const RunDims *__restrict__ d, int h
                    head ? hidden : uniform(d->output_dim), uniform(d->l2), head};
 }
 
-// Work item w = (item i, chunk k), over a grid-stride loop: the F32 sum, in
-// token order, of chunk k of item i's tokens (its live ones, when the item
-// has any live token; else all of them), and how many it summed. Tokens are
-// read 8 at a time (their loads in flight together), and added in order. A
-// row's CLS or LAST vector needs no sums.
-__global__ void __launch_bounds__(POOL_THREADS) pool_part_kernel(const RunDims *__restrict__ dims,
-                                                                 const float *__restrict__ x, int hidden, Packing p,
-                                                                 const int32_t *__restrict__ mask,
-                                                                 const uint32_t *__restrict__ ranges,
-                                                                 float *__restrict__ part, int32_t *__restrict__ cnt,
-                                                                 int chunks) {
+// Items of at most POOL_SHORT tokens (a token's or a sentence's range) are
+// summed by the finish itself; longer ones in chunks of POOL_CHUNK tokens,
+// work item w = (item i, chunk k) over a grid-stride loop in x, 256 columns a
+// workgroup in y. Each of POOL_WAVES waves sums POOL_SHORT tokens of the
+// chunk in token order, 16 bytes a lane and eight tokens' loads in flight,
+// and the waves' sums are added in order: F32 sums of the chunk's live tokens
+// (when the item has any; else of all of them), and how many.
+// (One workgroup a chunk over all columns, a chain of 256 tokens in 32
+// rounds of loads, left most of the chip idle: 64 us at 128 rows of 32-256
+// tokens x 384 where reading them takes 4; a part a wave made it 13. A
+// 5,500-token QA run's single-token ranges took 43 us there and 15 in the
+// finish.)
+// A row's CLS or LAST vector needs no sums.
+constexpr int POOL_SHORT = 32, POOL_WAVES = POOL_CHUNK / POOL_SHORT, POOL_COLS = 256;
+__global__ void __launch_bounds__(64 * POOL_WAVES) pool_part_kernel(const RunDims *__restrict__ dims,
+                                                                    const float *__restrict__ x, int hidden, Packing p,
+                                                                    const int32_t *__restrict__ mask,
+                                                                    const uint32_t *__restrict__ ranges,
+                                                                    float *__restrict__ part, int32_t *__restrict__ cnt,
+                                                                    int chunks) {
+    typedef float float4_v __attribute__((ext_vector_type(4)));
+    __shared__ float4_v sums[POOL_WAVES][64];
+    __shared__ int counts[POOL_WAVES];
     const PoolRun pr = pool_run(dims, hidden);
     if (pr.mode == 0 && pr.pooling != 1) return;
     const int seq = uniform(dims->seq), od = pr.od;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c = blockIdx.y * POOL_COLS + 4 * lane;   // this lane's four columns
+    if ((int)blockIdx.y * POOL_COLS >= od) return;
     for (int w = blockIdx.x; w < pr.items * chunks; w += gridDim.x) {
         const int i = w / chunks, k = w % chunks;
         int r, c0, c1;
         pool_span(i, pr.mode, p, ranges, r, c0, c1);
         const int cs = c0 + k * POOL_CHUNK;
-        if (cs >= c1) continue;   // past the item: the finish reads only its own chunks
-        const int ce = min(cs + POOL_CHUNK, c1), start = p.start[r];
+        if (c1 - c0 <= POOL_SHORT || cs >= c1) continue;   // the finish reads only its own chunks
+        const int start = p.start[r];
         const int32_t *mk = mask + (size_t)r * seq;
         int any = 0;
-        for (int q = c0 + (int)threadIdx.x; q < c1 && !any; q += POOL_THREADS) any = mk[q] != 0;
+        for (int q = c0 + (int)threadIdx.x; q < c1 && !any; q += 64 * POOL_WAVES) any = mk[q] != 0;
         const bool live_only = __syncthreads_or(any) != 0;
-        constexpr int MAXV = 8;
-        float acc[MAXV];
+        // This wave's tokens t0 + j, those to sum as bits.
+        const int t0 = cs + POOL_SHORT * wave;
+        const bool in = lane < POOL_SHORT && t0 + lane < c1;
+        const uint32_t use = (uint32_t)__ballot(in && (!live_only || mk[in ? t0 + lane : c0] != 0));
+        float4_v acc = {0, 0, 0, 0};
+        if (use && c < hidden) {
+            const float *col = x + (size_t)start * hidden + c;
+            for (int j0 = 0; j0 < POOL_SHORT; j0 += 8) {
+                float4_v v[8];
 #pragma unroll
-        for (int v = 0; v < MAXV; ++v) acc[v] = 0.0f;
-        int n = 0;
-        for (int q0 = cs; q0 < ce; q0 += 8) {
-            bool use[8];
-            float val[8][MAXV];
+                for (int j = 0; j < 8; ++j) v[j] = *(const float4_v *)(col + (size_t)min(t0 + j0 + j, c1 - 1) * hidden);
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int q = q0 + j;
-                use[j] = q < ce && (!live_only || mk[q] != 0);
-                const float *row = x + (size_t)(start + (use[j] ? q : cs)) * hidden;
-#pragma unroll
-                for (int v = 0; v < MAXV; ++v) {
-                    const int c = threadIdx.x + POOL_THREADS * v;
-                    val[j][v] = (use[j] && c < od) ? row[c] : 0.0f;
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                if (!use[j]) continue;
-#pragma unroll
-                for (int v = 0; v < MAXV; ++v) acc[v] = __fadd_rn(acc[v], val[j][v]);
-                ++n;
+                for (int j = 0; j < 8; ++j)
+                    if ((use >> (j0 + j)) & 1u) acc += v[j];
             }
         }
-        float *dst = part + ((size_t)i * chunks + k) * od;
+        sums[wave][lane] = acc;
+        if (lane == 0) counts[wave] = __popc(use);
+        __syncthreads();
+        if (wave == 0) {
+            float *dst = part + ((size_t)i * chunks + k) * od;
+            int n = counts[0];
 #pragma unroll
-        for (int v = 0; v < MAXV; ++v) {
-            const int c = threadIdx.x + POOL_THREADS * v;
-            if (c < od) dst[c] = acc[v];
+            for (int u = 1; u < POOL_WAVES; ++u) {
+                acc += sums[u][lane];
+                n += counts[u];
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (c + q < od) dst[c + q] = acc[q];
+            if (lane == 0 && blockIdx.y == 0) cnt[(size_t)i * chunks + k] = n;
         }
-        if (threadIdx.x == 0) cnt[(size_t)i * chunks + k] = n;
+        __syncthreads();   // sums is read before the next item writes it
     }
 }
 
-// Item i over a grid-stride loop: its vector from the chunk sums (or its
-// CLS or LAST row), then the cut and L2, or the span head.
+// Item i over a grid-stride loop: its vector from the chunk sums (a short
+// item's from its tokens, in token order; or its CLS or LAST row), then the
+// cut and L2, or the span head.
 __global__ void __launch_bounds__(POOL_THREADS) pool_kernel(const RunDims *__restrict__ dims,
                                                             const float *__restrict__ x, int hidden, Packing p,
+                                                            const int32_t *__restrict__ mask,
                                                             const uint32_t *__restrict__ ranges,
                                                             float *__restrict__ out, const float *__restrict__ hw,
                                                             const float *__restrict__ hb, int hout,
@@ -770,8 +792,34 @@ __global__ void __launch_bounds__(POOL_THREADS) pool_kernel(const RunDims *__res
                 const int c = threadIdx.x + POOL_THREADS * v;
                 if (c < od) acc[v] = x[(size_t)tok * hidden + c];
             }
+        } else if (c1 - c0 <= POOL_SHORT) {
+            const int32_t *mk = mask + (size_t)r * uniform(dims->seq);
+            const int lane = threadIdx.x & 63, len = c1 - c0;
+            const uint32_t all = (uint32_t)__ballot(lane < len), live = (uint32_t)__ballot(lane < len && mk[c0 + min(lane, len - 1)] != 0);
+            const uint32_t use = live ? live : all;
+            for (int j0 = 0; j0 < len; j0 += 4) {
+                float val[4][MAXV];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float *row = x + (size_t)(start + c0 + min(j0 + j, len - 1)) * hidden;
+#pragma unroll
+                    for (int v = 0; v < MAXV; ++v) {
+                        const int c = threadIdx.x + POOL_THREADS * v;
+                        val[j][v] = c < od ? row[c] : 0.0f;
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if (!((use >> (j0 + j)) & 1u)) continue;
+#pragma unroll
+                    for (int v = 0; v < MAXV; ++v) acc[v] = __fadd_rn(acc[v], val[j][v]);
+                }
+            }
+            const float inv = __fdiv_rn(1.0f, (float)__popc(use));
+#pragma unroll
+            for (int v = 0; v < MAXV; ++v) acc[v] = __fmul_rn(acc[v], inv);
         } else {
-            // The chunks' sums in chunk order (one chunk: its sum exactly).
+            // The chunks' sums in chunk order.
             const int nch = (c1 - c0 + POOL_CHUNK - 1) / POOL_CHUNK;
             int n = 0;
             for (int k = 0; k < nch; ++k) {
@@ -837,18 +885,18 @@ __global__ void __launch_bounds__(POOL_THREADS) pool_kernel(const RunDims *__res
 }
 
 // Workgroups a pooling launch takes at most: items beyond them loop.
-constexpr int POOL_GRID = 2048;
+constexpr int POOL_GRID = 8192;
 
 hipError_t pool(hipStream_t s, const RunDims *dims, int max_items, const float *x, int hidden, const Packing &p,
                 const int32_t *mask, const uint32_t *ranges, const PoolScratch &ps, float *out, const float *hw,
                 const float *hb, int hout) {
-    if (hidden > 8 * POOL_THREADS || hout < 0 || hout > HEAD_MAX) return hipErrorInvalidValue;
+    if (hidden > 8 * POOL_THREADS || hidden % 4 != 0 || hout < 0 || hout > HEAD_MAX) return hipErrorInvalidValue;
     if (max_items <= 0) return hipSuccess;
     if (!ps.part || !ps.cnt || ps.chunks <= 0) return hipErrorInvalidValue;
     const int part_blocks = (int)std::min<long>((long)max_items * ps.chunks, POOL_GRID);
-    enqueue(pool_part_kernel, dim3(part_blocks), dim3(POOL_THREADS), 0, s, dims, x, hidden, p, mask, ranges,
-            ps.part, ps.cnt, ps.chunks);
-    enqueue(pool_kernel, dim3(std::min(max_items, POOL_GRID)), dim3(POOL_THREADS), 0, s, dims, x, hidden, p,
+    enqueue(pool_part_kernel, dim3(part_blocks, (hidden + POOL_COLS - 1) / POOL_COLS), dim3(64 * POOL_WAVES), 0, s,
+            dims, x, hidden, p, mask, ranges, ps.part, ps.cnt, ps.chunks);
+    enqueue(pool_kernel, dim3(std::min(max_items, POOL_GRID)), dim3(POOL_THREADS), 0, s, dims, x, hidden, p, mask,
             ranges, out, hw, hb, hout, ps.part, ps.cnt, ps.chunks);
     return hipGetLastError();
 }
