@@ -1,12 +1,17 @@
 """The GEMM shapes for few rows (d32x32, 64x64), for F32 operands as BF16
 terms (x64x64, x128x128) and the rule that picks among them, at the edges of
-their tiles and of k, on an MI355X through the C ABI."""
+their tiles and of k, residual products in slices of K, and means of every
+length, on an MI355X through the C ABI."""
 import numpy as np
 import pytest
 
+import oracle
 import turboembed_amd as T
 from turboembed_amd import seam as S
-from turboembed_amd.model import to_bf16_bits
+from turboembed_amd.model import to_bf16_bits, with_dtype
+
+import small
+from test_gpu_parity import assert_close
 
 pytestmark = pytest.mark.gpu
 
@@ -73,3 +78,58 @@ def test_int8_shapes_have_the_same_bits(runtime, mnk):
     want = T.gemm_check(a, w, b, dtype=S.TURBO_DTYPE_I8, tile=7)
     for t in (0, 5, 21):
         np.testing.assert_array_equal(T.gemm_check(a, w, b, dtype=S.TURBO_DTYPE_I8, tile=t), want)
+
+
+@pytest.mark.parametrize("tier", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("family", ["bert", "modernbert"])
+@pytest.mark.parametrize("inter", [1536, 2080])
+def test_residual_products_in_slices_meet_the_oracle(context, monkeypatch, family, tier, inter):
+    # Short runs cut FFN-out's K into slices that the add + LayerNorm adds
+    # (2080: the last one shorter), from one token up; replayed and launched
+    # directly, the same bits.
+    build = getattr(small, family)
+    desc = build(seed=71, hidden=128, heads=2, inter=inter, positions=96, std=0.05)
+    precision = S.TURBO_PRECISION_EXACT if tier == "f32" else S.TURBO_PRECISION_FASTEST
+    if tier == "bf16":
+        desc, precision = with_dtype(desc, "bf16"), S.TURBO_PRECISION_MODEL
+    model = context.load(desc)
+    s = model.session(4, 96, precision)
+    monkeypatch.setenv("TURBO_ROCM_GRAPHS", "0")
+    direct = model.session(4, 96, precision)
+    for batch, seq in ((1, 1), (1, 33), (4, 96)):
+        ids, mask, types = small.ragged_rows(71 + seq, batch, seq, desc.vocab_size)
+        types = None if family == "modernbert" else types
+        got = s.embed(ids, mask, types)
+        assert_close(got, oracle.encode(desc, ids, mask, types), s.compute_dtype)
+        np.testing.assert_array_equal(direct.embed(ids, mask, types), got)
+    direct.close()
+    s.close()
+    model.close()
+
+
+def test_means_of_every_length_meet_the_oracle(context):
+    # Ranges at the edges of the finish's 32 tokens and of a chunk's parts and
+    # chunks, over masked tokens; a whole row's range the row's own mean bit for bit.
+    desc = small.bert(seed=73, hidden=320, heads=5, inter=64, positions=600, std=0.1)
+    g = np.random.Generator(np.random.PCG64(73))
+    ids = g.integers(0, desc.vocab_size, size=(3, 599)).astype(np.int32)
+    mask = np.ones((3, 599), np.int32)
+    mask[0, g.choice(np.arange(1, 598), 150, replace=False)] = 0
+    mask[0, 3] = 1
+    mask[1, 100:180] = 0
+    mask[2, 20:] = 0
+    types = np.zeros_like(ids)
+    lens = [1, 2, 31, 32, 33, 63, 64, 65, 255, 256, 257, 288, 289, 511, 512, 513]
+    ranges = [(r, 3 + r, 3 + r + n) for r in (0, 1) for n in lens]
+    ranges += [(1, 90, 110), (1, 60, 175), (2, 0, 20), (0, 0, 599)]
+    model = context.load(desc)
+    s = model.session(3, 600, S.TURBO_PRECISION_EXACT, max_ranges=len(ranges))
+    s.write_ranges(ids, mask, ranges, types)
+    s.run()
+    got = s.read()
+    assert_close(got, oracle.encode(desc, ids, mask, types, ranges=ranges), s.compute_dtype)
+    rows = s.embed(ids, mask, types)
+    np.testing.assert_array_equal(rows[0], got[-1])
+    np.testing.assert_array_equal(rows[2], got[-2])
+    s.close()
+    model.close()

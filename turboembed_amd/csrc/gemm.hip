@@ -1421,6 +1421,11 @@ template <typename T> constexpr Dt dt_of() {
     return sizeof(T) == 4 ? Dt::F32 : std::is_same<T, __bf16>::value ? Dt::BF16 : Dt::F16;
 }
 
+bool gemm_is_direct(Dt dt, int M, int N, int K, const EpiArgs &e) {
+    if (dt == Dt::I8 || M <= 0) return false;
+    return (dt != Dt::F32 && K % 64 == 0 ? pipelined_tile(M, N, K, e) : staged_tile(dt, M, N)) == 20;
+}
+
 template <typename T, int BK>
 static hipError_t gemm_t(hipStream_t s, const GemmRows &gr, int M, int N, int K, const void *A, int lda, const void *W,
                          const EpiArgs &e,

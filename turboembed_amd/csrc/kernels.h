@@ -123,6 +123,15 @@ hipError_t deberta_attention(hipStream_t s, Dt dt, const void *qkv, int tcap, in
 hipError_t layer_norm(hipStream_t s, const Span &sp, int max_tokens, int hidden, const float *in, const float *ln_w,
                       const float *ln_b, float eps, float *out_f32, void *out_h, Dt dt);
 
+// A residual product as the F32 sums of slices of its K, [slices][stride]
+// with rows of `hidden`, and the bias to add to them (NULL: none).
+struct SliceSum {
+    const float *ws = nullptr;
+    int slices = 0;   // 0: the product itself, in y
+    size_t stride = 0;
+    const float *bias = nullptr;
+};
+
 // The residual add and a LayerNorm in one pass, row by row: v = x + y (y in
 // ydt: F32, F16 or BF16). Post-norm (pre_norm 0): x = LN(v), and out_h =
 // LN(v) in `dt` when not NULL. Pre-norm (pre_norm 1): x = v, and out_h =
@@ -132,7 +141,8 @@ hipError_t layer_norm(hipStream_t s, const Span &sp, int max_tokens, int hidden,
 // Over the span's tokens; x, y and out_h point at the run's token 0.
 hipError_t add_layer_norm(hipStream_t s, const Span &sp, int max_tokens, int hidden, float *x, const void *y, Dt ydt,
                           const float *ln_w, const float *ln_b, float eps, int pre_norm, void *out_h, Dt dt,
-                          const QuantOut &qo = QuantOut(), bool res_h = false, bool keep_f32 = true);
+                          const QuantOut &qo = QuantOut(), bool res_h = false, bool keep_f32 = true,
+                          const SliceSum &sl = SliceSum());
 
 // What a GEMM does with each output once its sum is done.
 enum class Epi : int {
@@ -189,6 +199,11 @@ int gemm_tile_by_name(const char *s, size_t n);
 int gemm_candidates(Dt dt, int K, int lda, const EpiArgs &e, int *out, int cap);
 // The 256 x 384 block shape (8 waves of 128 x 96): a split run's products' shape.
 constexpr int WIDE_TILE = 15;
+// The slices of K a residual product (Bias epilogue) of at most M rows is best
+// cut into (1: none), and its launch: slice y's F32 sums at ws + y stride.
+int gemm_slices_of(Dt dt, int M, int N, int K, const EpiArgs &e);
+hipError_t gemm_slices(hipStream_t s, Dt dt, const Span &sp, int max_m, int N, int K, const void *A, int lda,
+                       const void *W, float *ws, int slices, size_t stride);
 // The block shape for a product that runs beside those of the run's other
 // parts, of at most M rows a part (0: the launcher's rule).
 int gemm_split_tile(Dt dt, int M, int N, int K, int parts, const EpiArgs &e);

@@ -298,11 +298,15 @@ __global__ void __launch_bounds__(256) layer_norm_kernel(Span sp, int hidden, co
 // The residual add and a LayerNorm in one pass (a wave a token): v = x + y,
 // then x = LN(v) (post-norm) or x = v (pre-norm), and out_h = LN(v). One
 // read of x and of the product, one write of x and of the operand copy.
-template <int G, typename Y, typename H, bool RES_H>
+constexpr int MAX_SLICES = 4;
+// SLICES: y is not read; the product is its slices' sum (sl), in slice order,
+// plus the bias, all of a row's reads in flight together.
+template <int G, typename Y, typename H, bool RES_H, bool SLICES = false>
 __global__ void __launch_bounds__(256) add_layer_norm_kernel(Span sp, int hidden, float *__restrict__ x,
                                                              const Y *__restrict__ y, const float *__restrict__ ln_w,
                                                              const float *__restrict__ ln_b, float eps, int pre_norm,
-                                                             int keep_f32, H *__restrict__ out_h, QuantOut qo) {
+                                                             int keep_f32, H *__restrict__ out_h, QuantOut qo,
+                                                             SliceSum sl = SliceSum()) {
     const Live lv = live_of(sp);
     const int local = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (local >= lv.tokens) return;
@@ -323,7 +327,25 @@ __global__ void __launch_bounds__(256) add_layer_norm_kernel(Span sp, int hidden
             // The residual: x, or (RES_H) the 16-bit rows the last norm wrote.
             if constexpr (RES_H) load4(hr + c, v[g]);
             else load4(row + c, v[g]);
-            load4(yr + c, a);
+            if constexpr (SLICES) {
+                const float *ws = sl.ws + (size_t)t * hidden + c;
+                float w[MAX_SLICES][4], b[4] = {0, 0, 0, 0};
+#pragma unroll
+                for (int u = 0; u < MAX_SLICES; ++u) {
+                    // (A slice past the last reads the first again, unused.)
+                    load4(ws + (u < sl.slices ? u * sl.stride : 0), w[u]);
+                }
+                if (sl.bias) load4(sl.bias + c, b);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    a[k] = w[0][k];
+#pragma unroll
+                    for (int u = 1; u < MAX_SLICES; ++u) a[k] = u < sl.slices ? a[k] + w[u][k] : a[k];
+                    a[k] += b[k];
+                }
+            } else {
+                load4(yr + c, a);
+            }
 #pragma unroll
             for (int k = 0; k < 4; ++k) v[g][k] = v[g][k] + a[k];
         } else {
@@ -423,7 +445,16 @@ constexpr int LN_ROWS = 2, LN_WAVES = 4, LN_FEW = 4096;
 template <typename H, int G, typename Y>
 static hipError_t add_ln_v(hipStream_t s, const Span &sp, int tokens, int hidden, float *x, const void *y,
                            const float *ln_w, const float *ln_b, float eps, int pre_norm, void *out_h,
-                           const QuantOut &qo, bool res_h, bool keep_f32) {
+                           const QuantOut &qo, bool res_h, bool keep_f32, const SliceSum &sl) {
+    if (sl.slices) {
+        if (res_h && sizeof(H) == 2)
+            enqueue((add_layer_norm_kernel<G, float, H, sizeof(H) == 2, true>), dim3((tokens + 3) / 4), dim3(256), 0, s,
+                    sp, hidden, x, (const float *)nullptr, ln_w, ln_b, eps, pre_norm, (int)keep_f32, (H *)out_h, qo, sl);
+        else
+            enqueue((add_layer_norm_kernel<G, float, H, false, true>), dim3((tokens + 3) / 4), dim3(256), 0, s, sp,
+                    hidden, x, (const float *)nullptr, ln_w, ln_b, eps, pre_norm, (int)keep_f32, (H *)out_h, qo, sl);
+        return hipGetLastError();
+    }
     // Two rows a wave on the 16-bit residual (measured: BERT-base's norms 6%
     // faster; on F32 rows, ModernBERT's, 2% slower). Other runs keep one
     // layout for all their norms: a layer read's final norm (layer_norm)
@@ -444,27 +475,27 @@ static hipError_t add_ln_v(hipStream_t s, const Span &sp, int tokens, int hidden
     }
     if (res_h && sizeof(H) == 2)
         enqueue((add_layer_norm_kernel<G, Y, H, sizeof(H) == 2>), dim3((tokens + 3) / 4), dim3(256), 0, s,
-                sp, hidden, x, (const Y *)y, ln_w, ln_b, eps, pre_norm, (int)keep_f32, (H *)out_h, qo);
+                sp, hidden, x, (const Y *)y, ln_w, ln_b, eps, pre_norm, (int)keep_f32, (H *)out_h, qo, sl);
     else
         enqueue((add_layer_norm_kernel<G, Y, H, false>), dim3((tokens + 3) / 4), dim3(256), 0, s, sp,
-                hidden, x, (const Y *)y, ln_w, ln_b, eps, pre_norm, (int)keep_f32, (H *)out_h, qo);
+                hidden, x, (const Y *)y, ln_w, ln_b, eps, pre_norm, (int)keep_f32, (H *)out_h, qo, sl);
     return hipGetLastError();
 }
 
 template <typename H, int G>
 static hipError_t add_ln_y(hipStream_t s, const Span &sp, int tokens, int hidden, float *x, const void *y, Dt ydt,
                            const float *ln_w, const float *ln_b, float eps, int pre_norm, void *out_h,
-                           const QuantOut &qo, bool res_h, bool keep_f32) {
+                           const QuantOut &qo, bool res_h, bool keep_f32, const SliceSum &sl) {
     switch (ydt) {
     case Dt::F16:
         return add_ln_v<H, G, _Float16>(s, sp, tokens, hidden, x, y, ln_w, ln_b, eps, pre_norm, out_h, qo, res_h,
-                                        keep_f32);
+                                        keep_f32, sl);
     case Dt::BF16:
         return add_ln_v<H, G, __bf16>(s, sp, tokens, hidden, x, y, ln_w, ln_b, eps, pre_norm, out_h, qo, res_h,
-                                      keep_f32);
+                                      keep_f32, sl);
     case Dt::F32:
         return add_ln_v<H, G, float>(s, sp, tokens, hidden, x, y, ln_w, ln_b, eps, pre_norm, out_h, qo, res_h,
-                                     keep_f32);
+                                     keep_f32, sl);
     default: return hipErrorInvalidValue;
     }
 }
@@ -590,8 +621,8 @@ static hipError_t ln_t(hipStream_t s, const Span &sp, int tokens, int hidden, co
 template <typename H>
 static hipError_t add_ln_t(hipStream_t s, const Span &sp, int tokens, int hidden, float *x, const void *y, Dt ydt,
                            const float *ln_w, const float *ln_b, float eps, int pre_norm, void *out_h,
-                           const QuantOut &qo, bool res_h, bool keep_f32) {
-    ROWWISE_DISPATCH(add_ln_y, s, sp, tokens, hidden, x, y, ydt, ln_w, ln_b, eps, pre_norm, out_h, qo, res_h, keep_f32)
+                           const QuantOut &qo, bool res_h, bool keep_f32, const SliceSum &sl) {
+    ROWWISE_DISPATCH(add_ln_y, s, sp, tokens, hidden, x, y, ydt, ln_w, ln_b, eps, pre_norm, out_h, qo, res_h, keep_f32, sl)
 }
 
 hipError_t embed_ln(hipStream_t s, const Span &sp, int max_tokens, int hidden, const int32_t *ids,
@@ -615,7 +646,7 @@ hipError_t embed_ln(hipStream_t s, const Span &sp, int max_tokens, int hidden, c
 
 hipError_t add_layer_norm(hipStream_t s, const Span &sp, int max_tokens, int hidden, float *x, const void *y, Dt ydt,
                           const float *ln_w, const float *ln_b, float eps, int pre_norm, void *out_h, Dt dt,
-                          const QuantOut &qo, bool res_h, bool keep_f32) {
+                          const QuantOut &qo, bool res_h, bool keep_f32, const SliceSum &sl) {
     if (max_tokens <= 0) return hipSuccess;
     if (qo.q && (dt != Dt::F16 || !out_h || hidden % 4 != 0)) return hipErrorInvalidValue;
     // A 16-bit residual is a post-norm's, read from and written to out_h.
@@ -624,13 +655,15 @@ hipError_t add_layer_norm(hipStream_t s, const Span &sp, int max_tokens, int hid
     switch (dt) {
     case Dt::F16:
         return add_ln_t<_Float16>(s, sp, max_tokens, hidden, x, y, ydt, ln_w, ln_b, eps, pre_norm, out_h, qo, res_h,
-                                  keep_f32);
+                                  keep_f32, sl);
     case Dt::BF16:
         return add_ln_t<__bf16>(s, sp, max_tokens, hidden, x, y, ydt, ln_w, ln_b, eps, pre_norm, out_h, qo, res_h,
-                                keep_f32);
+                                keep_f32, sl);
+    if (sl.slices < 0 || sl.slices > MAX_SLICES || (sl.slices && (!sl.ws || hidden % 4 != 0 || sl.stride % 4 != 0)))
+        return hipErrorInvalidValue;
     default:
         return add_ln_t<float>(s, sp, max_tokens, hidden, x, y, ydt, ln_w, ln_b, eps, pre_norm, out_h, qo, res_h,
-                               keep_f32);
+                               keep_f32, sl);
     }
 }
 

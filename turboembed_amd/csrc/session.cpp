@@ -1265,6 +1265,23 @@ static void run_layers(Session &s, hipStream_t st, int part, const Bounds &bd, T
         }
         LAUNCH(NAMES[g], gemm(st, s.dt, sp, T, lg.N, lg.K, A, lg.K, a_tok, lg.W, lg.e, bc.tile[g]));
     };
+    // The out or FFN-out product of layer l for the add + LayerNorm after it:
+    // into y, or, where the rule cuts it into slices of K (few rows), as their
+    // sums in the split-K workspace.
+    auto mm_residual = [&](uint32_t l, GemmSlot g) {
+        SliceSum sl;
+        if (bc.tile[g] == 0 && splitk_fits(s, bd.bin, g)) {
+            const LayerGemm lg = layer_gemm(s, l, g);
+            const int n = gemm_slices_of(s.dt, T, lg.N, lg.K, lg.e);
+            if (n > 1) {
+                sl = SliceSum{s.splitk_ws, n, (size_t)T * lg.N, lg.e.bias};
+                LAUNCH(NAMES[g], gemm_slices(st, s.dt, sp, T, lg.N, lg.K, lg.A, lg.K, lg.W, s.splitk_ws, n, sl.stride));
+                return sl;
+            }
+        }
+        mm(l, g);
+        return sl;
+    };
     // The out or FFN-out product of layer l with its residual add and the
     // norm (w, b) in its epilogue, when the bin's choice for it is the
     // whole-row shape: whether it ran so. (F16 post-norm sessions alone,
@@ -1323,13 +1340,13 @@ static void run_layers(Session &s, hipStream_t st, int part, const Bounds &bd, T
         // Post-norm: x = LN1(x + y), in the product's epilogue on the
         // whole-row shape. Pre-norm: x += y, xh = LN_mlp(x).
         if (!mm_ln(l, G_OUT, L.ln1_w, L.ln1_b, !res_h)) {
-            mm(l, G_OUT);
+            const SliceSum sl = mm_residual(l, G_OUT);
             if (m.modern)
-                LAUNCH("add_layer_norm",
-                       add_layer_norm(st, sp, T, H, s.x, s.y, s.ydt, L.ln2_w, nullptr, m.eps, 1, norm_out, dt, qo));
+                LAUNCH("add_layer_norm", add_layer_norm(st, sp, T, H, s.x, s.y, s.ydt, L.ln2_w, nullptr, m.eps, 1,
+                                                        norm_out, dt, qo, false, true, sl));
             else
                 LAUNCH("add_layer_norm", add_layer_norm(st, sp, T, H, s.x, s.y, s.ydt, L.ln1_w, L.ln1_b, m.eps, 0,
-                                                        norm_out, dt, qo, res_h, !res_h));
+                                                        norm_out, dt, qo, res_h, !res_h, sl));
         }
         aq_ready = i8;
         mm(l, G_FFN1);
@@ -1340,16 +1357,16 @@ static void run_layers(Session &s, hipStream_t st, int part, const Bounds &bd, T
         // the last layer, and after a layer whose ranges are read.
         const bool keep_f32 = !res_h || l + 1 == nl || (reads > 1 && l + reads >= nl);
         if (!mm_ln(l, G_FFN2, L.ln2_w, L.ln2_b, keep_f32)) {
-            mm(l, G_FFN2);
+            const SliceSum sl = mm_residual(l, G_FFN2);
             if (!m.modern)
                 LAUNCH("add_layer_norm", add_layer_norm(st, sp, T, H, s.x, s.y, s.ydt, L.ln2_w, L.ln2_b, m.eps, 0,
-                                                        norm_out, dt, next, res_h, keep_f32));
+                                                        norm_out, dt, next, res_h, keep_f32, sl));
             else if (l + 1 < nl)
                 LAUNCH("add_layer_norm", add_layer_norm(st, sp, T, H, s.x, s.y, s.ydt, m.ls[l + 1].ln1_w, nullptr,
-                                                        m.eps, 1, norm_out, dt, next));
+                                                        m.eps, 1, norm_out, dt, next, false, true, sl));
             else
-                LAUNCH("add_layer_norm",
-                       add_layer_norm(st, sp, T, H, s.x, s.y, s.ydt, m.final_w, nullptr, m.eps, 0, nullptr, dt));
+                LAUNCH("add_layer_norm", add_layer_norm(st, sp, T, H, s.x, s.y, s.ydt, m.final_w, nullptr, m.eps, 0,
+                                                        nullptr, dt, QuantOut(), false, true, sl));
         }
         aq_ready = i8 && l + 1 < nl;
         if (reads > 1 && l + 1 < nl && l + reads >= nl) {
