@@ -133,7 +133,7 @@ struct SliceSum {
 };
 
 // The residual add and a LayerNorm in one pass, row by row: v = x + y (y in
-// ydt: F32, F16 or BF16). Post-norm (pre_norm 0): x = LN(v), and out_h =
+// ydt: F32, F16 or BF16; or the slices' sum). Post-norm (pre_norm 0): x = LN(v), and out_h =
 // LN(v) in `dt` when not NULL. Pre-norm (pre_norm 1): x = v, and out_h =
 // LN(v) in `dt` (out_h F32 on the F32 tier). ln_b NULL is no bias.
 // A post-norm on 16-bit rows may carry its residual in them (res_h): v =

@@ -25,10 +25,9 @@ __global__ void __launch_bounds__(1024) pack_rows_kernel(const int32_t *__restri
     // Each wave takes whole rows: every lane's last live column among its
     // strided ones, then the wave's maximum (no atomics on a few shared words).
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
-    // (Rows of a multiple of 4 columns are read 16 bytes a lane, 256 columns
-    // a wave a step; a wave's four rows at a time, their reads issued
-    // together.)
-    typedef int int4_t __attribute__((ext_vector_type(4)));
+    // (Rows are read 16 bytes a lane from any column's boundary, 256 columns a
+    // wave a step; a wave's four rows at a time, their reads issued together.)
+    typedef int int4_t __attribute__((ext_vector_type(4), aligned(4)));
     constexpr int RW = 4;
     for (int r0 = wave; r0 < batch; r0 += RW * waves) {
         int last[RW];
@@ -38,15 +37,13 @@ __global__ void __launch_bounds__(1024) pack_rows_kernel(const int32_t *__restri
             last[j] = 0;
             if (r >= batch) continue;
             const int32_t *row = mask + (size_t)r * seq;
-            if ((seq & 3) == 0) {
+            // (A row's last read may run past it, into the next row or the
+            // plane after the mask's.)
 #pragma unroll 4
-                for (int c = 4 * lane; c < seq; c += 256) {
-                    const int4_t v = *(const int4_t *)(row + c);
-                    last[j] = v[3] ? c + 4 : v[2] ? c + 3 : v[1] ? c + 2 : v[0] ? c + 1 : last[j];
-                }
-            } else {
-                for (int c = lane; c < seq; c += 64)
-                    if (row[c] != 0) last[j] = c + 1;
+            for (int c = 4 * lane; c < seq; c += 256) {
+                const int4_t v = *(const int4_t *)(row + c);
+                const int n = seq - c;
+                last[j] = v[3] && n > 3 ? c + 4 : v[2] && n > 2 ? c + 3 : v[1] && n > 1 ? c + 2 : v[0] ? c + 1 : last[j];
             }
         }
 #pragma unroll
@@ -59,15 +56,25 @@ __global__ void __launch_bounds__(1024) pack_rows_kernel(const int32_t *__restri
         }
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
+    // The first wave's scan, 64 rows at a time (one thread's chain over 128
+    // rows took a third of the launch).
+    if (wave == 0) {
         int t = 0;
-        for (int r = 0; r < batch; ++r) {
-            const int l = lens[r];
-            p.start[r] = t;
-            p.len[r] = l;
-            t += l;
+        for (int r0 = 0; r0 < batch; r0 += 64) {
+            const int r = r0 + lane, l = r < batch ? lens[r] : 0;
+            int sum = l;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int v = __shfl_up(sum, o, 64);
+                if (lane >= o) sum += v;
+            }
+            if (r < batch) {
+                p.start[r] = t + sum - l;
+                p.len[r] = l;
+            }
+            t += __shfl(sum, 63, 64);
         }
-        p.tokens[0] = t;
+        if (lane == 0) p.tokens[0] = t;
     }
 }
 
@@ -652,6 +659,8 @@ hipError_t add_layer_norm(hipStream_t s, const Span &sp, int max_tokens, int hid
     // A 16-bit residual is a post-norm's, read from and written to out_h.
     if (res_h && (dt == Dt::F32 || !out_h || pre_norm)) return hipErrorInvalidValue;
     if (!keep_f32 && !res_h) return hipErrorInvalidValue;
+    if (sl.slices < 0 || sl.slices > MAX_SLICES || (sl.slices && (!sl.ws || hidden % 4 != 0 || sl.stride % 4 != 0)))
+        return hipErrorInvalidValue;
     switch (dt) {
     case Dt::F16:
         return add_ln_t<_Float16>(s, sp, max_tokens, hidden, x, y, ydt, ln_w, ln_b, eps, pre_norm, out_h, qo, res_h,
@@ -659,8 +668,6 @@ hipError_t add_layer_norm(hipStream_t s, const Span &sp, int max_tokens, int hid
     case Dt::BF16:
         return add_ln_t<__bf16>(s, sp, max_tokens, hidden, x, y, ydt, ln_w, ln_b, eps, pre_norm, out_h, qo, res_h,
                                 keep_f32, sl);
-    if (sl.slices < 0 || sl.slices > MAX_SLICES || (sl.slices && (!sl.ws || hidden % 4 != 0 || sl.stride % 4 != 0)))
-        return hipErrorInvalidValue;
     default:
         return add_ln_t<float>(s, sp, max_tokens, hidden, x, y, ydt, ln_w, ln_b, eps, pre_norm, out_h, qo, res_h,
                                keep_f32, sl);
@@ -693,6 +700,10 @@ hipError_t layer_norm(hipStream_t s, const Span &sp, int max_tokens, int hidden,
 // the core's host head, core/src/qa/session.rs:268-276, sums the same terms).
 constexpr int POOL_THREADS = 256;
 
+__device__ __forceinline__ uint64_t uniform64(uint64_t v) {
+    return (uint64_t)(uint32_t)uniform((int)(v >> 32)) << 32 | (uint32_t)uniform((int)(uint32_t)v);
+}
+
 // Item i's tokens: a row's live extent (mode 0) or a range within it.
 __device__ __forceinline__ void pool_span(int i, int mode, const Packing &p, const uint32_t *__restrict__ ranges, int &r,
                                           int &c0, int &c1) {
@@ -721,7 +732,7 @@ __device__ __forceinline__ PoolRun pool_run(const RunDims *__restrict__ d, int h
 
 // Items of at most POOL_SHORT tokens (a token's or a sentence's range) are
 // summed by the finish itself; longer ones in chunks of POOL_CHUNK tokens,
-// work item w = (item i, chunk k) over a grid-stride loop in x, 256 columns a
+// work item w = (chunk k, item i) over a grid-stride loop in x, 256 columns a
 // workgroup in y. Each of POOL_WAVES waves sums POOL_SHORT tokens of the
 // chunk in token order, 16 bytes a lane and eight tokens' loads in flight,
 // and the waves' sums are added in order: F32 sums of the chunk's live tokens
@@ -748,50 +759,73 @@ __global__ void __launch_bounds__(64 * POOL_WAVES) pool_part_kernel(const RunDim
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c = blockIdx.y * POOL_COLS + 4 * lane;   // this lane's four columns
     if ((int)blockIdx.y * POOL_COLS >= od) return;
-    for (int w = blockIdx.x; w < pr.items * chunks; w += gridDim.x) {
-        const int i = w / chunks, k = w % chunks;
-        int r, c0, c1;
-        pool_span(i, pr.mode, p, ranges, r, c0, c1);
-        const int cs = c0 + k * POOL_CHUNK;
-        if (c1 - c0 <= POOL_SHORT || cs >= c1) continue;   // the finish reads only its own chunks
-        const int start = p.start[r];
-        const int32_t *mk = mask + (size_t)r * seq;
-        int any = 0;
-        for (int q = c0 + (int)threadIdx.x; q < c1 && !any; q += 64 * POOL_WAVES) any = mk[q] != 0;
-        const bool live_only = __syncthreads_or(any) != 0;
-        // This wave's tokens t0 + j, those to sum as bits.
-        const int t0 = cs + POOL_SHORT * wave;
-        const bool in = lane < POOL_SHORT && t0 + lane < c1;
-        const uint32_t use = (uint32_t)__ballot(in && (!live_only || mk[in ? t0 + lane : c0] != 0));
-        float4_v acc = {0, 0, 0, 0};
-        if (use && c < hidden) {
-            const float *col = x + (size_t)start * hidden + c;
-            for (int j0 = 0; j0 < POOL_SHORT; j0 += 8) {
-                float4_v v[8];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) v[j] = *(const float4_v *)(col + (size_t)min(t0 + j0 + j, c1 - 1) * hidden);
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    if ((use >> (j0 + j)) & 1u) acc += v[j];
-            }
+    // A workgroup's work items, every gridDim.x-th from its own (chunk k of
+    // items 0, 1, ..., then chunk k + 1's): each thread looks whether one has
+    // tokens for this kernel, so a run of single-token ranges costs one look.
+    const int total = pr.items * chunks;
+    __shared__ uint64_t todo[POOL_WAVES];
+    for (int base = blockIdx.x; base < total; base += 64 * POOL_WAVES * gridDim.x) {
+        const int mine = base + (int)(threadIdx.x * gridDim.x);
+        bool has = mine < total;
+        if (has) {
+            int r, c0, c1;
+            pool_span(mine % pr.items, pr.mode, p, ranges, r, c0, c1);
+            has = c1 - c0 > POOL_SHORT && c0 + mine / pr.items * POOL_CHUNK < c1;
         }
-        sums[wave][lane] = acc;
-        if (lane == 0) counts[wave] = __popc(use);
+        const uint64_t b = __ballot(has);
+        __syncthreads();   // the last round's todo has been read
+        if (lane == 0) todo[wave] = b;
         __syncthreads();
-        if (wave == 0) {
-            float *dst = part + ((size_t)i * chunks + k) * od;
-            int n = counts[0];
-#pragma unroll
-            for (int u = 1; u < POOL_WAVES; ++u) {
-                acc += sums[u][lane];
-                n += counts[u];
+        for (int u = 0; u < 64 * POOL_WAVES; ++u) {
+            const uint64_t left = uniform64(todo[u >> 6]) >> (u & 63);
+            if (left == 0) {
+                u |= 63;
+                continue;
             }
+            u += __builtin_ctzll(left);
+            const int w = base + u * (int)gridDim.x, i = w % pr.items, k = w / pr.items;
+            int r, c0, c1;
+            pool_span(i, pr.mode, p, ranges, r, c0, c1);
+            const int cs = c0 + k * POOL_CHUNK;
+            const int start = p.start[r];
+            const int32_t *mk = mask + (size_t)r * seq;
+            int any = 0;
+            for (int q = c0 + (int)threadIdx.x; q < c1 && !any; q += 64 * POOL_WAVES) any = mk[q] != 0;
+            const bool live_only = __syncthreads_or(any) != 0;
+            // This wave's tokens t0 + j, those to sum as bits.
+            const int t0 = cs + POOL_SHORT * wave;
+            const bool in = lane < POOL_SHORT && t0 + lane < c1;
+            const uint32_t use = (uint32_t)__ballot(in && (!live_only || mk[in ? t0 + lane : c0] != 0));
+            float4_v acc = {0, 0, 0, 0};
+            if (use && c < hidden) {
+                const float *col = x + (size_t)start * hidden + c;
+                for (int j0 = 0; j0 < POOL_SHORT; j0 += 8) {
+                    float4_v v[8];
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-                if (c + q < od) dst[c + q] = acc[q];
-            if (lane == 0 && blockIdx.y == 0) cnt[(size_t)i * chunks + k] = n;
+                    for (int j = 0; j < 8; ++j) v[j] = *(const float4_v *)(col + (size_t)min(t0 + j0 + j, c1 - 1) * hidden);
+#pragma unroll
+                    for (int j = 0; j < 8; ++j)
+                        if ((use >> (j0 + j)) & 1u) acc += v[j];
+                }
+            }
+            sums[wave][lane] = acc;
+            if (lane == 0) counts[wave] = __popc(use);
+            __syncthreads();
+            if (wave == 0) {
+                float *dst = part + ((size_t)i * chunks + k) * od;
+                int n = counts[0];
+#pragma unroll
+                for (int u = 1; u < POOL_WAVES; ++u) {
+                    acc += sums[u][lane];
+                    n += counts[u];
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (c + q < od) dst[c + q] = acc[q];
+                if (lane == 0 && blockIdx.y == 0) cnt[(size_t)i * chunks + k] = n;
+            }
+            __syncthreads();   // sums is read before the next item writes it
         }
-        __syncthreads();   // sums is read before the next item writes it
     }
 }
 
@@ -918,7 +952,7 @@ __global__ void __launch_bounds__(POOL_THREADS) pool_kernel(const RunDims *__res
 }
 
 // Workgroups a pooling launch takes at most: items beyond them loop.
-constexpr int POOL_GRID = 8192;
+constexpr int POOL_GRID = 8192, POOL_PARTS = 1024;
 
 hipError_t pool(hipStream_t s, const RunDims *dims, int max_items, const float *x, int hidden, const Packing &p,
                 const int32_t *mask, const uint32_t *ranges, const PoolScratch &ps, float *out, const float *hw,
@@ -926,7 +960,7 @@ hipError_t pool(hipStream_t s, const RunDims *dims, int max_items, const float *
     if (hidden > 8 * POOL_THREADS || hidden % 4 != 0 || hout < 0 || hout > HEAD_MAX) return hipErrorInvalidValue;
     if (max_items <= 0) return hipSuccess;
     if (!ps.part || !ps.cnt || ps.chunks <= 0) return hipErrorInvalidValue;
-    const int part_blocks = (int)std::min<long>((long)max_items * ps.chunks, POOL_GRID);
+    const int part_blocks = (int)std::min<long>((long)max_items * ps.chunks, POOL_PARTS);
     enqueue(pool_part_kernel, dim3(part_blocks, (hidden + POOL_COLS - 1) / POOL_COLS), dim3(64 * POOL_WAVES), 0, s,
             dims, x, hidden, p, mask, ranges, ps.part, ps.cnt, ps.chunks);
     enqueue(pool_kernel, dim3(std::min(max_items, POOL_GRID)), dim3(POOL_THREADS), 0, s, dims, x, hidden, p, mask,
