@@ -353,8 +353,12 @@ class Session:
         [count, output_dim] (turbo_embed_write_layer_ranges; the core's
         checks, tokens.rs:99-130, 153-215)."""
         head = self.model.desc.span_head
-        ranges = list(ranges)
-        if not ranges:
+        # (An integer array [n, 3] is taken as it lies in memory, wrapped to 32
+        # bits as the fields of a triple are: 5,500 triples one by one are
+        # 2 ms of Python.)
+        if not (isinstance(ranges, np.ndarray) and ranges.dtype.kind in "iu" and ranges.shape[1:] == (3,)):
+            ranges = list(ranges)
+        if not len(ranges):
             raise TurboError(S.TURBO_E_INVALID_ARGUMENT, 0, "count is 0: a run needs at least one range")
         if layers == 0:
             raise TurboError(S.TURBO_E_INVALID_ARGUMENT, 9, "layers 0: a range write needs at least 1 layer")
@@ -379,9 +383,13 @@ class Session:
         if head is not None:
             r.head, r.output_dim = 1, head[0].shape[0]
         r.taps, r.tap_alone = layers, 1 if alone else 0
-        arr = (S.turbo_token_range * max(1, len(ranges)))()
-        for i, (row, start, end) in enumerate(ranges):
-            arr[i].row, arr[i].start, arr[i].end = row, start, end
+        if isinstance(ranges, np.ndarray):
+            triples = np.ascontiguousarray(ranges).astype(np.uint32, casting="unsafe")
+            arr = triples.ctypes.data_as(C.POINTER(S.turbo_token_range))
+        else:
+            arr = (S.turbo_token_range * max(1, len(ranges)))()
+            for i, (row, start, end) in enumerate(ranges):
+                arr[i].row, arr[i].start, arr[i].end = row, start, end
         err = S.new_error()
         mask = self._keep[1]
         _ok(self.lib.turbo_rocm_check_ranges(r.batch, r.seq, r.seq, _i32(mask), arr, len(ranges), self.max_ranges,

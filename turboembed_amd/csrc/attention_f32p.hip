@@ -84,11 +84,11 @@ __global__ void __launch_bounds__(64 * F32P_WAVES) attention_f32p_kernel(const T
         k_hi = min(len, qw + 32 + window);
     }
 
-    // A lane's columns of K and Q: with F32 operands half h's D / 2, one a
-    // product step; else 8 of each 16. Its key of K: the MFMA row itself, or,
+    // A lane's columns of K and Q: 16 bytes of each 32, its half's (with F32
+    // operands a column a product step). Its key of K: the MFMA row itself, or,
     // so that P's registers hold runs of 8 keys, with bits 2 and 3 exchanged.
-    constexpr int KSTEP = F32 ? VEC : 16;
-    const int kcol = F32 ? h * (D / 2) : h * 8;
+    constexpr int KSTEP = 2 * VEC;
+    const int kcol = h * VEC;
     const int krow = F32 ? ql : (ql & ~12) | ((ql & 4) << 1) | ((ql & 8) >> 1);
     vec q[KV];
 #pragma unroll

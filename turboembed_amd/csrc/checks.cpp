@@ -91,21 +91,22 @@ int32_t turbo_rocm_check_ranges(uint32_t batch, uint32_t seq, uint32_t row_strid
     const uint32_t stride = row_stride == 0 ? seq : row_stride;
     for (uint32_t i = 0; i < count; ++i) {
         const turbo_token_range g = ranges[i];
-        const std::string at = "ranges[" + std::to_string(i) + "]: ";
+        // (The message's start, made for a refused range alone.)
+        const auto at = [i] { return "ranges[" + std::to_string(i) + "]: "; };
         if (g.row >= batch)
             return refuse(err, TURBO_E_INVALID_ARGUMENT,
-                          at + "row " + std::to_string(g.row) + " is not under batch " + std::to_string(batch));
+                          at() + "row " + std::to_string(g.row) + " is not under batch " + std::to_string(batch));
         if (g.start >= g.end)
             return refuse(err, TURBO_E_INVALID_ARGUMENT,
-                          at + "start " + std::to_string(g.start) + " is not under end " + std::to_string(g.end));
+                          at() + "start " + std::to_string(g.start) + " is not under end " + std::to_string(g.end));
         if (g.end > seq)
             return refuse(err, TURBO_E_INVALID_ARGUMENT,
-                          at + "end " + std::to_string(g.end) + " is over seq " + std::to_string(seq));
+                          at() + "end " + std::to_string(g.end) + " is over seq " + std::to_string(seq));
         bool live = false;
         for (uint32_t p = g.start; p < g.end && !live; ++p) live = mask[(size_t)g.row * stride + p] == 1;
         if (!live)
             return refuse(err, TURBO_E_UNSUPPORTED_OPTION,
-                          at + "columns " + std::to_string(g.start) + " to " + std::to_string(g.end) + " of row " +
+                          at() + "columns " + std::to_string(g.start) + " to " + std::to_string(g.end) + " of row " +
                               std::to_string(g.row) +
                               " hold no token whose mask is 1, and the rocm backend does not compute mask-0 columns");
     }

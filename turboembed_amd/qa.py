@@ -30,11 +30,16 @@ def span_logits(session, windows, fill_id=0):
         ids = np.full((len(chunk), seq), fill_id, np.int32)
         types = np.zeros_like(ids)
         mask = np.zeros_like(ids)
-        ranges = []
+        # Every live token's own range, row by row.
+        ranges = np.empty((sum(len(w) for w, _ in chunk), 3), np.uint32)
+        k = 0
         for r, (wi, wt) in enumerate(chunk):
             n = len(wi)
             ids[r, :n], types[r, :n], mask[r, :n] = wi, wt, 1
-            ranges += [(r, i, i + 1) for i in range(n)]
+            ranges[k:k + n, 0] = r
+            ranges[k:k + n, 1] = np.arange(n)
+            ranges[k:k + n, 2] = np.arange(1, n + 1)
+            k += n
         session.write_ranges(ids, mask, ranges, types, normalize=S.TURBO_NORMALIZE_NONE)
         session.run()
         logits = session.read()
