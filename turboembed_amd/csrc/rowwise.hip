@@ -739,9 +739,9 @@ __device__ __forceinline__ PoolRun pool_run(const RunDims *__restrict__ d, int h
 // (when the item has any; else of all of them), and how many.
 // (One workgroup a chunk over all columns, a chain of 256 tokens in 32
 // rounds of loads, left most of the chip idle: 64 us at 128 rows of 32-256
-// tokens x 384 where reading them takes 4; a part a wave made it 13. A
+// tokens x 384 where reading them takes 6; a part a wave makes it 8. A
 // 5,500-token QA run's single-token ranges took 43 us there and 15 in the
-// finish.)
+// finish, and take 9 and 18.)
 // A row's CLS or LAST vector needs no sums.
 constexpr int POOL_SHORT = 32, POOL_WAVES = POOL_CHUNK / POOL_SHORT, POOL_COLS = 256;
 __global__ void __launch_bounds__(64 * POOL_WAVES) pool_part_kernel(const RunDims *__restrict__ dims,
