@@ -9,7 +9,7 @@
 // F64 adds took 38 ms for at 128 rows of 768, 15 times the encoder's run;
 // here it takes 48 us, on 16 x 16 tiles of (row, output), a thread each, both
 // operands through LDS 64 columns at a time, bound by the F64 chain's latency
-// at six workgroups' waves a CU; the call is 3400 us.
+// at one or two workgroups a CU; the call is 3400 us.
 #include "kernels.h"
 #include "launch.h"
 #include "devmath.h"
