@@ -133,3 +133,15 @@ def test_means_of_every_length_meet_the_oracle(context):
     np.testing.assert_array_equal(rows[2], got[-2])
     s.close()
     model.close()
+
+
+def test_a_model_without_layers_opens_with_split_bins(context):
+    # Embeddings alone, on a session whose larger bins split their runs: the
+    # split's rule has no layer to take its products' sizes from.
+    desc = small.bert(seed=79, layers=0, positions=512)
+    ids, mask, types = small.ragged_rows(79, 24, 512, desc.vocab_size)
+    model = context.load(desc)
+    s = model.session(64, 512, S.TURBO_PRECISION_EXACT)
+    assert_close(s.embed(ids, mask, types), oracle.encode(desc, ids, mask, types), s.compute_dtype)
+    s.close()
+    model.close()

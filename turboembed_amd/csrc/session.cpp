@@ -875,6 +875,7 @@ static Bounds bounds_of(const Session &s, int b, uint32_t parts) {
 // its residual products' tiles are too few (16,384 tokens: 128 at N = 768).
 static void split_defaults(Session &s) {
     const Model &m = *s.model;
+    if (m.ls.empty()) return;   // embeddings alone: no products
     for (int b = 0; b < s.kc.bins; ++b) {
         const uint32_t parts = parts_of_bin(s, b);
         if (parts < 2) continue;
