@@ -72,6 +72,25 @@ def test_operands_of_every_magnitude_keep_their_terms(runtime):
         assert np.abs(got.astype(np.float64) / sa[:, None] / sw[None, :] - want).max() <= 1e-5 * np.sqrt(k)
 
 
+@pytest.mark.parametrize("tile", [22, 23])
+def test_values_that_are_not_finite_are_the_f32_core_s(runtime, tile):
+    # Infinities, a NaN, F32's largest value and sums past it, one to a row or
+    # column in tiles of their own and shared ones: where the F32 matrix core
+    # has an infinity, a NaN or a value, the BF16 terms have the same.
+    m, n, k = 300, 260, 100
+    a, w, b = _operands(m, n, k)
+    big = np.finfo(np.float32).max
+    a[3, 7], a[40, 99], a[41, 0], a[41, 50] = np.inf, -np.inf, np.inf, -np.inf
+    a[130, 5], a[280, 64] = np.nan, big
+    a[200], a[200, 3], w[:, 3] = 0.0, 2.0 ** 126, 4.0 * w[:, 3]   # products past F32's range, one a sum
+    w[70, 3], w[255, 98] = -np.inf, np.nan
+    w[10] = 2.0 ** -100
+    with np.errstate(all="ignore"):
+        got, want = T.gemm_check(a, w, b, tile=tile), T.gemm_check(a, w, b, tile=1)
+    assert np.isinf(want).any(1)[[3, 40, 200, 280]].all() and np.isfinite(want[[200, 280], 10]).all()
+    np.testing.assert_allclose(got, want, rtol=1e-4, atol=1e-4)
+
+
 @pytest.mark.parametrize("mnk", [(1, 64, 128), (65, 192, 384), (300, 2304, 768)])
 def test_int8_shapes_have_the_same_bits(runtime, mnk):
     a, w, b = _operands(*mnk)

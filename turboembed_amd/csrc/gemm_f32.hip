@@ -8,8 +8,9 @@
 // 2^-24 that each of an F32 sum's roundings may be off, and the sum of the x0
 // w0 products rounds once per 16 columns of k where the F32 MFMA's rounds
 // once per two (error against 64 bits at K = 768: see the test).
-// (Finite operands; an infinity gives NaN, as the norm after every product
-// of the encoder would make of it.)
+// An infinite or NaN operand's terms differ by NaN, so its sums are NaN here
+// whatever the product comes to; and a sum may pass F32's range: a wave with a
+// sum that is not finite takes its tiles again on the F32 matrix core.
 //
 // A workgroup of WM x WN waves per BM x BN output tile. K advances BK columns
 // a stage: while one is multiplied, the next one's F32 operands, loaded during
@@ -45,6 +46,22 @@ __device__ __forceinline__ void split2(float x, float y, uint32_t (&t)[3]) {
     t[1] = __builtin_bit_cast(uint32_t, bf16x2{(__bf16)x1, (__bf16)y1});
     const float x2 = x1 - __uint_as_float(t[1] << 16), y2 = y1 - __uint_as_float(t[1] & 0xffff0000u);
     t[2] = __builtin_bit_cast(uint32_t, bf16x2{(__bf16)x2, (__bf16)y2});
+}
+
+// A 32 x 32 tile on the F32 matrix core, a lane's row of each operand straight
+// from memory: four columns of each eight, its half's (K a multiple of 4).
+__device__ __forceinline__ floatx16 f32_tile(const float *a, const float *w, int K) {
+    const int h = (threadIdx.x & 63) >> 5;
+    floatx16 v{};
+#pragma unroll 1
+    for (int k0 = 0; k0 < K; k0 += 8) {
+        const int k = k0 + 4 * h;
+        const f32x4 x = k < K ? *(const f32x4 *)(a + k) : f32x4{0, 0, 0, 0};
+        const f32x4 y = k < K ? *(const f32x4 *)(w + k) : f32x4{0, 0, 0, 0};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v = Mma<float>::run(x[q], y[q], v);
+    }
+    return v;
 }
 
 template <int BM, int BN, int WM, int WN, int BK, Epi KIND>
@@ -154,14 +171,29 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_f32_split_kernel(Span sp, i
         }
         __syncthreads();
     }
+    float z = 0.0f;   // 0 as long as every sum is finite
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
             acc[i][j] += low[i][j];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) z = fmaf(acc[i][j][r], 0.0f, z);
+        }
+    if (__ballot(z != 0.0f) != 0) {   // uniform
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+                acc[i][j] = f32_tile(A + (size_t)min(m0 + wm * (BM / WM) + i * 32 + (lane & 31), M - 1) * lda,
+                                     W + (size_t)min(n0 + wn * (BN / WN) + j * 32 + (lane & 31), N - 1) * K, K);
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
             epilogue_tile<float, KIND>(e, M, N, m0 + wm * (BM / WM) + i * 32, n0 + wn * (BN / WN) + j * 32 + (lane & 31),
                                        acc[i][j]);
-        }
 }
 
 template <int BM, int BN, int WM, int WN, int BK>
