@@ -72,6 +72,23 @@ def test_operands_of_every_magnitude_keep_their_terms(runtime):
         assert np.abs(got.astype(np.float64) / sa[:, None] / sw[None, :] - want).max() <= 1e-5 * np.sqrt(k)
 
 
+@pytest.mark.parametrize("value", [1 + 2.0 ** -7 - 2.0 ** -16, 1 + 2.0 ** -8 - 2.0 ** -17, 1 + 2.0 ** -8 + 2.0 ** -17])
+@pytest.mark.parametrize("k", [16, 64, 768])
+def test_bf16_terms_of_like_operands_lose_no_more_than_a_rounding(runtime, value, k):
+    # Every product the same, so that what the six products leave out (at most
+    # 2^-24 of each) and the roundings (one per 16 columns of k, one as the
+    # small terms' sum, 2^-7 of the whole with five roundings per 16, is
+    # added) may all go one way.
+    x = np.float32(value)
+    a, w = np.full((70, k), x), np.full((90, k), x)
+    a[1::2] *= -1
+    want = a.astype(np.float64) @ w.astype(np.float64).T
+    bound = (2 + k / 16 * (1 + 5 / 128)) * 2.0 ** -24
+    for tile in (22, 23):
+        off = np.abs(T.gemm_check(a, w, tile=tile) / want - 1).max()
+        assert off <= bound, (tile, off * 2 ** 24)
+
+
 @pytest.mark.parametrize("tile", [22, 23])
 def test_values_that_are_not_finite_are_the_f32_core_s(runtime, tile):
     # Infinities, a NaN, F32's largest value and sums past it, one to a row or

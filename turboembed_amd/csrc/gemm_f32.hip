@@ -1,13 +1,19 @@
 // The F32 tier's large products on the BF16 matrix cores. The F32 MFMA
 // (v_mfma_f32_32x32x2f32) runs at a sixteenth of the BF16 one's rate, so each
-// F32 operand is taken as the sum of three BF16 terms, x = x0 + x1 + x2
-// exactly (8 bits of the significand each: x0 cut off, x1 and x2 rounded to
-// the nearest), and a product as the six terms' products of order 2^-16 and
-// above, x0 w0 + x0 w1 + x1 w0 + x0 w2 + x1 w1 + x2 w0, summed in F32, the five small ones apart from
-// the first. What is left out is of order 2^-26 of each product, against the
-// 2^-24 that each of an F32 sum's roundings may be off, and the sum of the x0
-// w0 products rounds once per 16 columns of k where the F32 MFMA's rounds
-// once per two (error against 64 bits at K = 768: see the test).
+// F32 operand is taken as the sum of three BF16 terms, each rounded to the
+// nearest of what the ones before it left, x = x0 + x1 + x2 exactly (the
+// split of Henry, Tang and Heinecke, "Leveraging the bfloat16 Artificial
+// Intelligence Datatype For Higher-Precision Computations", 2019), and a
+// product as the six largest of its terms' products, x0 w0 + x0 w1 + x1 w0 +
+// x0 w2 + x1 w1 + x2 w0, summed in F32, the five small ones apart from the
+// first. |x1| is at most 2^-8 of x's power of two and |x2| 2^-17, so what is
+// left out, x1 w2 + x2 w1 + x2 w2, is at most 2^-24 of a product (2^-27.4 in
+// the root mean square over normal operands), what one rounding of an F32 sum
+// may be off by; with x0 cut off instead, x1 is up to 2^-7, of x's own sign,
+// and up to 2^-22 is left out (products 1% faster). And
+// the sum of the x0 w0 products rounds once per 16 columns of k where the F32
+// MFMA's rounds once per two. (From |x| = 2^-103 up: a smaller one's last
+// term falls below BF16's normal range.)
 // An infinite or NaN operand's terms differ by NaN, so its sums are NaN here
 // whatever the product comes to; and a sum may pass F32's range: a wave with a
 // sum that is not finite takes its tiles again on the F32 matrix core.
@@ -15,16 +21,17 @@
 // A workgroup of WM x WN waves per BM x BN output tile. K advances BK columns
 // a stage: while one is multiplied, the next one's F32 operands, loaded during
 // the stage before, are split and stored to the other LDS buffer and the
-// loads of the one after it go out; one barrier a stage. A row of each term's LDS plane is padded by 16 bytes, so
-// that the 16-byte fragment reads of consecutive rows fall in distinct banks.
+// loads of the one after it go out; one barrier a stage. A row of each term's
+// LDS plane is padded by 16 bytes, so that the 16-byte fragment reads of
+// consecutive rows fall in distinct banks.
 //
 // Measured (us at 4096 rows, N x K; the F32 MFMA on 128 x 128 tiles, which
-// all F32 products took, then on 64 x 64): 768 x 768 here 47 against 66 and
-// 55; 2304 x 768 131 (242, 152); 768 x 3072 146 (266, 187); 384 x 1536 56
-// (142, 74). A stage's vector work, LDS traffic (six reads and three writes
+// all F32 products took, then on 64 x 64): 768 x 768 here 46 against 81 and
+// 54; 2304 x 768 134 (242, 150); 768 x 3072 144 (262, 184); 384 x 1536 54
+// (139, 73). A stage's vector work, LDS traffic (six reads and three writes
 // of a term per element) and products take about a third of its time each
 // and a single workgroup's do not overlap: the 128 x 128 tile runs eight
-// waves, not four (768 x 3072: 146 against 190), and 64 x 64 tiles two
+// waves, not four (768 x 3072: 144 against 190), and 64 x 64 tiles two
 // workgroups a CU. BK 16, and the scheduler told to interleave the three,
 // were no faster.
 #include "kernels.h"
@@ -40,9 +47,8 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 // Two values' three terms, a pair a word.
 __device__ __forceinline__ void split2(float x, float y, uint32_t (&t)[3]) {
-    const uint32_t xu = __float_as_uint(x), yu = __float_as_uint(y);
-    t[0] = __builtin_amdgcn_perm(yu, xu, 0x07060302);   // the high halves
-    const float x1 = x - __uint_as_float(xu & 0xffff0000u), y1 = y - __uint_as_float(yu & 0xffff0000u);
+    t[0] = __builtin_bit_cast(uint32_t, bf16x2{(__bf16)x, (__bf16)y});
+    const float x1 = x - __uint_as_float(t[0] << 16), y1 = y - __uint_as_float(t[0] & 0xffff0000u);
     t[1] = __builtin_bit_cast(uint32_t, bf16x2{(__bf16)x1, (__bf16)y1});
     const float x2 = x1 - __uint_as_float(t[1] << 16), y2 = y1 - __uint_as_float(t[1] & 0xffff0000u);
     t[2] = __builtin_bit_cast(uint32_t, bf16x2{(__bf16)x2, (__bf16)y2});
@@ -66,8 +72,9 @@ __device__ __forceinline__ floatx16 f32_tile(const float *a, const float *w, int
 
 template <int BM, int BN, int WM, int WN, int BK, Epi KIND>
 __global__ void __launch_bounds__(64 * WM * WN) gemm_f32_split_kernel(Span sp, int a_tok, int N, int K,
-                                                             const float *__restrict__ A, int lda,
-                                                             const float *__restrict__ W, EpiArgs e, int grid_n) {
+                                                                      const float *__restrict__ A, int lda,
+                                                                      const float *__restrict__ W, EpiArgs e,
+                                                                      int grid_n) {
     constexpr int RS = BK * 2 + 16;              // bytes of an LDS row
     constexpr int PLANE = (BM + BN) * RS, BUF = 3 * PLANE;
     constexpr int THREADS = 64 * WM * WN;
@@ -203,8 +210,8 @@ static hipError_t launch(hipStream_t s, const GemmRows &gr, int M, int N, int K,
     constexpr int bytes = 2 * 3 * (BM + BN) * (BK * 2 + 16);
 #define SPLIT_CASE(E)                                                                                               \
     case Epi::E:                                                                                                    \
-        enqueue((gemm_f32_split_kernel<BM, BN, WM, WN, BK, Epi::E>), dim3(gn * gm), dim3(64 * WM * WN), bytes, s, gr.sp, gr.a_tok, N, \
-                K, (const float *)A, lda, (const float *)W, e, gn);                                                 \
+        enqueue((gemm_f32_split_kernel<BM, BN, WM, WN, BK, Epi::E>), dim3(gn * gm), dim3(64 * WM * WN), bytes, s,   \
+                gr.sp, gr.a_tok, N, K, (const float *)A, lda, (const float *)W, e, gn);                             \
         return hipGetLastError();
     switch (e.kind) {
         SPLIT_CASE(Plain)
