@@ -86,9 +86,12 @@ int32_t turbo_rocm_rerank_scores(const float *states, uint32_t n, uint32_t hidde
 /* turbo_rocm_rerank_run: the windows of `pairs` pairs ([windows, seq] ids and
  * types, each window's length, and the pair it belongs to) through a
  * TURBO_TASK_RERANK session of this backend, max_batch windows a run, as
- * CLS rows at full width with no normalization, then the head above; each
- * pair's score is the largest of its windows' (core/src/session/rerank.rs:
- * 111-219). pairs may not exceed the session's max_batch. */
+ * CLS rows at full width with no normalization, then the head above, computed
+ * on the device with its tensors copied there on every call (the same F64
+ * products; the classifier's sum in another order, so a score may be an F32
+ * rounding off the host's); each pair's score is the largest of its windows'
+ * (core/src/session/rerank.rs:111-219). pairs may not exceed the session's
+ * max_batch. */
 int32_t turbo_rocm_rerank_run(void *session, const int32_t *ids, const int32_t *types, const uint32_t *lengths,
                               uint32_t windows, uint32_t seq, const uint32_t *owner, uint32_t pairs,
                               const float *pooler_weight, const float *pooler_bias, const float *classifier_weight,

@@ -1,9 +1,10 @@
 // The sequence classification head over a rerank run's CLS states, beside
 // them on the device: the pooler's dense rows and the classifier's one row
 // (reference core/src/session/rerank.rs:166-191) with F64 products and sums,
-// each rounded to F32 once, as the host head (rerank.cpp) computes them. Its
-// F64 sums run in tile order, not column order: the scores differ by F32
-// roundings of values F64's last bits apart.
+// each rounded to F32 once, as the host head (rerank.cpp) computes them. A
+// product of two F32 values is exact in F64, and a pooler's sum runs from its
+// bias in column order, so it has the host's bits; the classifier's is summed
+// by the lanes of a wave, F64's last bits off the host's.
 //
 // The pooler is hidden^2 products a row, which one host thread's chain of
 // F64 adds took 38 ms for at 128 rows of 768, 15 times the encoder's run;
@@ -25,7 +26,7 @@ __global__ void __launch_bounds__(256) rerank_pooler_kernel(const float *__restr
     __shared__ float xs[HEAD_TILE][HEAD_COLS + 1], ws[HEAD_TILE][HEAD_COLS + 1];
     const int o0 = blockIdx.x * HEAD_TILE, r0 = blockIdx.y * HEAD_TILE;
     const int o = threadIdx.x % HEAD_TILE, r = threadIdx.x / HEAD_TILE;
-    double sum = 0.0;
+    double sum = b && o0 + o < hidden ? (double)b[o0 + o] : 0.0;
     for (int k0 = 0; k0 < hidden; k0 += HEAD_COLS) {
         __syncthreads();
         for (int i = threadIdx.x; i < HEAD_TILE * HEAD_COLS; i += 256) {
@@ -38,7 +39,7 @@ __global__ void __launch_bounds__(256) rerank_pooler_kernel(const float *__restr
         for (int k = 0; k < HEAD_COLS; ++k) sum = fma((double)ws[o][k], (double)xs[r][k], sum);
     }
     if (r0 + r < rows && o0 + o < hidden)
-        pooled[(size_t)(r0 + r) * hidden + o0 + o] = (float)tanh(sum + (b ? (double)b[o0 + o] : 0.0));
+        pooled[(size_t)(r0 + r) * hidden + o0 + o] = (float)tanh(sum);
 }
 
 // A wave a row: its logit, and whether its state was finite.

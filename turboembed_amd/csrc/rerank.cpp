@@ -1,8 +1,10 @@
-// The rerank caller of the encoder, on the host: pair windows over token ids,
-// the runs that encode them through the backend's table, and the sequence
-// classification head. Restates the reference core's caller side
-// (core/src/tokenizer/pair.rs:27-99, core/src/session/rerank.rs:111-219),
-// which the encoder path serves with CLS rows at full width, unnormalized.
+// The rerank caller of the encoder, on the host: pair windows over token ids
+// and the runs that encode them through the backend's table, each run's rows
+// scored beside them on the device (head.hip), and the sequence
+// classification head over states that the caller holds. Restates the
+// reference core's caller side (core/src/tokenizer/pair.rs:27-99,
+// core/src/session/rerank.rs:111-219), which the encoder path serves with CLS
+// rows at full width, unnormalized.
 #include <cmath>
 #include <cstring>
 #include <limits>
