@@ -44,7 +44,9 @@ def test_small_and_split_shapes_match_numpy(runtime, dtype, tile, mnk):
     want = _rounded(a, dtype) @ _rounded(w, dtype).T + b
     # An F32 sum of k products of unit variance: k roundings of at most
     # 2^-24 of a partial sum (at most about 5 sqrt(k)) if every one went
-    # the same way; they do not, and a tenth of that bounds them.
+    # the same way; they do not, and a tenth of that bounds them. (Every
+    # shape's, the F32 core's 1.7e-5 at k = 100 too; a BF16 term's product
+    # left out would pass here, and fails the two tests of the terms below.)
     bound = max(0.1 * k * 5 * np.sqrt(k) * 2.0 ** -24, 4e-6)
     assert np.abs(got - want).max() <= bound, (np.abs(got - want).max(), bound)
 
@@ -52,7 +54,7 @@ def test_small_and_split_shapes_match_numpy(runtime, dtype, tile, mnk):
 @pytest.mark.parametrize("mnk", [(200, 300, 772), (300, 256, 3072)])
 def test_bf16_terms_are_no_further_off_than_the_f32_products(runtime, mnk):
     # Against 64 bits: three BF16 terms an operand, six products, must not
-    # lose to the F32 matrix core's own sums (measured 3.2e-7 against 9.2e-7
+    # lose to the F32 matrix core's own sums (measured 3.4e-7 against 1.0e-6
     # at k = 3072).
     a, w, b = _operands(*mnk)
     want = a.astype(np.float64) @ w.astype(np.float64).T + b

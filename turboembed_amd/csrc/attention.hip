@@ -803,11 +803,10 @@ __global__ void __launch_bounds__(256) deberta_attention_kernel(const T *__restr
 // token) scores 0 against every position of the row: the mean of their
 // values.
 template <typename T>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) deberta_attention_mfma_kernel(const T *__restrict__ qkv, int tcap, int heads, Span sp,
-                                                           int nqb, Packing p, const int32_t *__restrict__ mask,
-                                                           const T *__restrict__ pos,
-                                                           const int32_t *__restrict__ buckets, int positions,
-                                                           T *__restrict__ ctx) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+deberta_attention_mfma_kernel(const T *__restrict__ qkv, int tcap, int heads, Span sp, int nqb, Packing p,
+                              const int32_t *__restrict__ mask, const T *__restrict__ pos,
+                              const int32_t *__restrict__ buckets, int positions, T *__restrict__ ctx) {
     constexpr int D = 64, QB = 128;
     typedef typename AttnMma<T>::frag frag;
     typedef uint32_t vec4 __attribute__((ext_vector_type(4)));

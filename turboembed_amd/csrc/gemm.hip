@@ -1376,7 +1376,11 @@ static int pipelined_tile(int M, int N, int K, const EpiArgs &e) {
             tile = t;
         }
     };
-    // (One round of 32 x 32 tiles: 768 x 3072 at 24 rows 12 us against 13.)
+    // One round of 32 x 32 tiles: within 5% of 64 x 64 either way up to 256
+    // rows (us, 24 rows: N = 768 5.4 against 5.7, 768 x 3072 12.5 against 13.0;
+    // 256 rows: 5.9 against 5.8, 13.8 against 13.2), and the shape whose
+    // residual products go to the add + LayerNorm in slices of K. Past a
+    // round it loses: N = 2304 at 128 rows 8.6 against 6.0.
     if (rounds(M, N, 32, 32, cus) <= 1 && !gemm_made_to_fail(20)) return 20;
     if ((!qkv || e.hidden % 96 == 0) && (K >= 2048 || r192 <= 1)) take(13, 3.7 * 1.03 * r192);
     take(5, 2.1 * rounds(M, N, 128, 128, cus));
@@ -1384,6 +1388,21 @@ static int pipelined_tile(int M, int N, int K, const EpiArgs &e) {
     return tile;
 }
 
+// A product beside those of the run's other parts: 256 x 384 tiles, or 256 x
+// 192 where those leave the part's share of the compute units idle. Times a
+// round as in pipelined_tile (256 x 192 3.7, 256 x 384 5.9, a launch alone at
+// K = 768 20 to 24 us and 33 to 37 against 64 x 64's 5.8), over fractions of a
+// round past the first, since another part's tiles fill a part's last one,
+// and a tenth in 256 x 384's favour, whose waves read a third less LDS a
+// product. Whole runs in us, two parts, 256 x 192 against 256 x 384: where the
+// rule takes 256 x 192, BERT-base (4 layers) of 5,472 tokens out 772 (807), FFN-out 773
+// (906), of 9,344 992 (1,031), 993 (1,130), of 16,192 1,493 (1,464), 1,500
+// (1,547), MiniLM (6) of 7,120 963 (1,002), 962 (1,067), ModernBERT (4) of
+// 10,800 1,029 (1,061), 1,027 (1,077); where it does not, BERT-base of 9,344
+// Q/K/V 1,009 (990), FFN-in 1,062 (991), of 25,984 out 2,250 (2,223), FFN-in
+// 2,307 (2,217). The rule sees the bin's largest part, so a run of few of its
+// bin's tokens may lose by it: MiniLM's Q/K/V of 7,120 781 (963), XLM-R's (2
+// layers) FFN-out of 7,200 677 (754).
 int gemm_split_tile(Dt dt, int M, int N, int K, int parts, const EpiArgs &e) {
     const double at_once = std::max(1, cu_count() / parts);
     auto cost = [&](double round, int bm, int bn) {
@@ -1415,8 +1434,8 @@ static int staged_tile(Dt dt, int M, int N) {
 // Block shapes by number: 1-3 and 14 stage operands through registers (any K
 // a multiple of 8, and the F32 tier); 20 shares K among its waves (the same
 // operands); 22 and 23 take F32 operands as BF16 terms; 4-13, 15, 16 and 21
-// are the pipelined kernel, for 16-bit operands with K a multiple of 64 (every encoder shape
-// here).
+// are the pipelined kernel, for 16-bit operands with K a multiple of 64 (every
+// encoder shape here).
 template <typename T> constexpr Dt dt_of() {
     return sizeof(T) == 4 ? Dt::F32 : std::is_same<T, __bf16>::value ? Dt::BF16 : Dt::F16;
 }
@@ -1440,7 +1459,8 @@ static hipError_t gemm_t(hipStream_t s, const GemmRows &gr, int M, int N, int K,
     }
     if (gemm_made_to_fail(tile)) return hipErrorInvalidDeviceFunction;
     // A pipelined shape asked of an operand it cannot take runs the staged kernel.
-    if (((tile >= 4 && tile <= 13) || tile == 15 || tile == 16 || tile == 21) && !pipelined) tile = (N % 128 == 0 && M >= 8192) ? 2 : 1;
+    if (((tile >= 4 && tile <= 13) || tile == 15 || tile == 16 || tile == 21) && !pipelined)
+        tile = (N % 128 == 0 && M >= 8192) ? 2 : 1;
     // Q, K and V must each start on a wave's column boundary: a shape whose
     // waves are wider than 64 columns runs 64-column waves (K = hidden is a
     // multiple of 64 on the pipelined kernel) when they do not.
@@ -1488,7 +1508,13 @@ static hipError_t gemm_t(hipStream_t s, const GemmRows &gr, int M, int N, int K,
 }
 
 // The rule's block shape on 128-byte int8 rows: as pipelined_tile, every shape
-// having the same bits.
+// having the same bits. Half the stages a product make a round shorter and the
+// shapes less far apart (us at K = 768: 64 x 64 5.1, 128 x 128 9.0, 256 x 256
+// 17.5, so 1 to 1.8 to 3.4), but the shape it picks is the fastest or within
+// 2% at 64 to 4,096 rows (us 64 x 64, 128 x 128, 256 x 256): 1,024 rows at N =
+// 768 5.6, 9.3, 17.6, at 2304 12.9, 10.3, 18.5; 2,048 rows at 3072 28.5, 22.5,
+// 22.7; 4,096 rows at 2304 45.5, 32.2, 24.1. At 8,192 rows it takes 128 x 128
+// for 768 x 3072, 45.9 against 43.0.
 static int i8_tile(int M, int N) {
     const long cus = cu_count();
     const double wide = 4.3 * rounds(M, N, 256, 256, cus), mid = 2.1 * rounds(M, N, 128, 128, cus),

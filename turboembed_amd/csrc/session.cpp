@@ -702,8 +702,9 @@ Session *session_open(Model *m, const turbo_backend_session_desc *desc, turbo_ba
     // Rows, the run's dimensions and the ranges in one allocation, in the
     // staging buffer's order: the ids, mask and types planes, then (on a
     // 64-byte boundary) the dimensions, the ranges right after them.
-    // (Each plane starts on 16 bytes: the packing kernel reads a row's mask
-    // 16 bytes a lane when the run's seq is a multiple of 4.)
+    // (The packing kernel reads a row's mask 16 bytes a lane, up to three
+    // columns past the row: past the last row they are the types plane's,
+    // which has to follow the mask's in this allocation.)
     const size_t plane = plane_ints(*s);
     const size_t dims_at = (3 * plane + 15) / 16 * 16;
     s->staging_ints = dims_at + sizeof(RunDims) / 4 + 3 * (size_t)s->max_ranges;
@@ -872,7 +873,8 @@ static Bounds bounds_of(const Session &s, int b, uint32_t parts) {
 // ModernBERT 16 x 2048-8192 45.4-45.6 ms against 45.4-46.6 (timing whole
 // runs in the tuner could not tell them apart reliably: its short bursts run
 // at clocks a sustained run does not). In the le16k bin, and at hidden 384,
-// its residual products' tiles are too few (16,384 tokens: 128 at N = 768).
+// its residual products' tiles are too few (16,384 tokens: 128 at N = 768;
+// gemm_split_tile has both sides).
 static void split_defaults(Session &s) {
     const Model &m = *s.model;
     if (m.ls.empty()) return;   // embeddings alone: no products
