@@ -28,7 +28,7 @@
 // (a lane a query, its keys read from LDS one by one), us a launch: F16 heads
 // of 32, 128 rows of 32-256 tokens in two parts side by side 35 against 187;
 // F32 heads of 32, 32 rows of 16-128, 16 against 45; F32 heads of 64, 24 rows
-// of 33-300, 101 against 316. Short rows wait for memory (each wave has eight
+// of 33-300, 94 to 101 against 316. Short rows wait for memory (each wave has eight
 // blocks at most there), F32 heads of 64 for the F32 matrix cores and the
 // 32-byte pieces in which their rows are read.
 #include <type_traits>
