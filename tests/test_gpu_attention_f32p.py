@@ -47,3 +47,25 @@ def test_rows_at_block_edges_meet_the_oracle(context, tier, heads, family, windo
     assert np.array_equal(s.embed(ids, mask, types), got)
     s.close()
     model.close()
+
+
+@pytest.mark.parametrize("heads", [4, 2])
+@pytest.mark.parametrize("family", ["bert", "modernbert"])
+@pytest.mark.parametrize("scale", [1e4, 1e6])
+def test_scores_of_any_size_meet_the_oracle(context, heads, family, scale):
+    # Query and key weights scaled by 1e4 and 1e6: scores of 1e9 and 1e13,
+    # whose ulps are far past exp's range, so all weight is on one key (or on
+    # equal ones) and only the scores' differences may count.
+    desc = getattr(small, family)(seed=51, hidden=128, heads=heads, inter=64, positions=200, std=0.2)
+    for i, t in enumerate(desc.tensors):
+        if family == "bert" and i >= 5 and (i - 5) % 16 in (0, 2):
+            desc.tensors[i] = t * np.float32(scale)
+        if family == "modernbert" and i >= 3 and (i - 3) % 6 == 1:
+            desc.tensors[i][:256] *= np.float32(scale)
+    ids, mask, types = small.ragged_rows(3, 6, 150, desc.vocab_size)
+    types = None if family == "modernbert" else types
+    model = context.load(desc)
+    s = model.session(6, 150, S.TURBO_PRECISION_EXACT)
+    assert_close(s.embed(ids, mask, types), oracle.encode(desc, ids, mask, types), s.compute_dtype)
+    s.close()
+    model.close()

@@ -9,9 +9,10 @@
 // computed, and the waves of a (row, head) pair meet in the caches. Scores
 // are computed transposed, S^T = K Q^T, so a lane holds one query (lane % 32)
 // and 16 of the block's keys, the other 16 in the lane 32 away; the online
-// softmax runs in F32 in base 2 with the scale and the maximum taken in one
-// fused multiply-add, and moves its maximum only when a score passes it by
-// more than 2^8. The context is computed transposed too, O^T += V^T P^T, from
+// softmax runs in F32 in base 2, on a score's distance from the maximum (the
+// difference first, then the scale: the product less a rounded maximum is off
+// by half its ulp, past exp2's range from scores of 1e9 on), and moves its
+// maximum only when a score passes it by more than 2^8. The context is computed transposed too, O^T += V^T P^T, from
 // P as the score registers hold it:
 // - F32 operands: v_mfma_f32_32x32x2f32 for both products, register r of P
 //   against the four-key groups of V^T that its keys lie in.
@@ -28,9 +29,9 @@
 // (a lane a query, its keys read from LDS one by one), us a launch: F16 heads
 // of 32, 128 rows of 32-256 tokens in two parts side by side 35 against 187;
 // F32 heads of 32, 32 rows of 16-128, 16 against 45; F32 heads of 64, 24 rows
-// of 33-300, 94 to 101 against 316. Short rows wait for memory (each wave has eight
-// blocks at most there), F32 heads of 64 for the F32 matrix cores and the
-// 32-byte pieces in which their rows are read.
+// of 33-300, 94 to 101 against 316. Short rows wait for memory (each wave has
+// eight blocks at most there), F32 heads of 64 for the F32 matrix cores and
+// the 32-byte pieces in which their rows are read.
 #include <type_traits>
 
 #include "kernels.h"
@@ -126,7 +127,7 @@ __global__ void __launch_bounds__(64 * F32P_WAVES) attention_f32p_kernel(const T
 #pragma unroll
     for (int t = 0; t < NO; ++t) o[t] = floatx16{};
     float m_run = -INFINITY, lsum = 0.0f;
-    const float scale = 1.4426950408889634f / sqrtf((float)D);
+    const float scale = 1.4426950408889634f / sqrtf((float)D), rescale = RESCALE / scale;
 
     auto step = [&](Block &b, int kb) {
         if (kb >= k_hi) return;   // uniform
@@ -169,20 +170,20 @@ __global__ void __launch_bounds__(64 * F32P_WAVES) attention_f32p_kernel(const T
         float mx = sc[0];
 #pragma unroll
         for (int i = 1; i < 16; ++i) mx = fmaxf(mx, sc[i]);
-        mx = halves_max(mx) * scale;
-        if (__ballot(mx > m_run + RESCALE) != 0) {
+        mx = halves_max(mx);
+        if (__ballot(mx > m_run + rescale) != 0) {
             const float m_new = fmaxf(m_run, mx);
-            const float f = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_new);
+            const float f = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m_run - m_new) * scale);
 #pragma unroll
             for (int t = 0; t < NO; ++t) o[t] *= f;
             lsum *= f;
             m_run = m_new;
         }
-        const float sub = m_run == -INFINITY ? 0.0f : BIAS - m_run;
+        const float m = m_run == -INFINITY ? 0.0f : m_run;
         float pr[16];
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-            pr[i] = __builtin_amdgcn_exp2f(fmaf(sc[i], scale, sub));
+            pr[i] = __builtin_amdgcn_exp2f(fmaf(sc[i] - m, scale, BIAS));
             lsum += pr[i];
         }
         if constexpr (F32) {
