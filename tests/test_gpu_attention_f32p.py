@@ -69,3 +69,15 @@ def test_scores_of_any_size_meet_the_oracle(context, heads, family, scale):
     assert_close(s.embed(ids, mask, types), oracle.encode(desc, ids, mask, types), s.compute_dtype)
     s.close()
     model.close()
+
+
+@pytest.mark.parametrize("heads", [4, 2])
+@pytest.mark.parametrize("window", [149, 150, 2 ** 31 - 156])
+def test_windows_over_the_rows_length_reach_every_key(context, heads, window):
+    desc = small.modernbert(seed=57, hidden=128, heads=heads, inter=64, positions=200, window=2 * window)
+    ids, mask, _ = small.ragged_rows(3, 6, 150, desc.vocab_size)
+    model = context.load(desc)
+    s = model.session(6, 150, S.TURBO_PRECISION_EXACT)
+    assert_close(s.embed(ids, mask), oracle.encode(desc, ids, mask, None), s.compute_dtype)
+    s.close()
+    model.close()

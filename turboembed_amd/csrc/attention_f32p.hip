@@ -237,6 +237,9 @@ bool attention_f32p_takes(Dt dt, int d) { return d == 32 ? dt != Dt::I8 : d == 6
 hipError_t attention_f32p(hipStream_t s, Dt dt, const void *qkv, int tcap, int heads, int d, const Packing &p,
                           const int32_t *mask, const Span &sp, int max_rows, int max_len, int window, void *ctx) {
     if (!attention_f32p_takes(dt, d)) return hipErrorInvalidValue;
+    // (A window over the rows' length is none, and the kernel's sums of a key
+    // and a window stay in range.)
+    if (window >= max_len) window = INT32_MAX;
     // A 1-D grid of groups of 8 (row, head) pairs times nqb query blocks.
     const int nqb = (max_len + 32 * F32P_WAVES - 1) / (32 * F32P_WAVES), pairs = heads * max_rows;
     const dim3 grid((pairs + 7) / 8 * 8 * nqb), block(64 * F32P_WAVES);
