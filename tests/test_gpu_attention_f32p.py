@@ -81,3 +81,36 @@ def test_windows_over_the_rows_length_reach_every_key(context, heads, window):
     assert_close(s.embed(ids, mask), oracle.encode(desc, ids, mask, None), s.compute_dtype)
     s.close()
     model.close()
+
+
+@pytest.mark.parametrize("tier, heads, value", [("f32", h, v) for h in (4, 2) for v in (np.inf, -np.inf, np.nan)] +
+                         [("f16", 4, np.inf), ("f16", 4, -np.inf)])
+def test_a_head_of_infinite_or_nan_scores_has_no_context(context, tier, heads, value):
+    # One key column of head 1 infinite (a weight or a bias; on F16 a bias
+    # past its range): each query's scores are infinities of either sign, the
+    # largest infinite or all of them minus infinity. Or not a number. The
+    # head then gives what one of zero values gives, in the first layer alone.
+    width, at = 128 // heads, 128 // heads + 5
+    value16 = np.copysign(1e6, value) if tier == "f16" else value
+
+    def model_with(what):
+        # (Layer 0's key weight and bias are tensors 7 and 8, its value ones 9 and 10.)
+        desc = small.bert(seed=58, hidden=128, heads=heads, inter=64, positions=300, std=0.1, layers=2)
+        if what == "zero values":
+            desc.tensors[9][width:2 * width], desc.tensors[10][width:2 * width] = 0.0, 0.0
+        elif what == "weight":
+            desc.tensors[7][at, 3] = value
+        else:
+            desc.tensors[8][at] = value16
+        return desc
+
+    desc = model_with("zero values")
+    ids, mask, types = small.ragged_rows(4, 9, 300, desc.vocab_size)
+    want = oracle.encode(desc, ids, mask, types)
+    precision = S.TURBO_PRECISION_EXACT if tier == "f32" else S.TURBO_PRECISION_FASTEST
+    for what in ("bias",) if tier == "f16" else ("weight", "bias"):
+        model = context.load(model_with(what))
+        s = model.session(9, 300, precision)
+        assert_close(s.embed(ids, mask, types), want, s.compute_dtype)
+        s.close()
+        model.close()

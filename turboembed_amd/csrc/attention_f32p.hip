@@ -23,7 +23,9 @@
 //   2^-32 of a query's largest.
 // A key that is not live (masked, outside the window, past the row) scores
 // minus infinity and its V reads as 0, so nothing of it reaches a live query;
-// a query with no live key gets a zero context.
+// a query with no live key gets a zero context. So does one whose largest
+// score is infinite, and a score that is not a number weighs 0 (queries or
+// keys past the operand type's range).
 //
 // Measured against the scalar kernel of attention.hip, which these heads took
 // (a lane a query, its keys read from LDS one by one), us a launch: F16 heads
@@ -49,6 +51,14 @@ __device__ __forceinline__ float halves_sum(float v) {
 __device__ __forceinline__ float halves_max(float v) {
     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+// (By the value's bits, and behind the compiler's back: this source is built
+// without NaNs.)
+__device__ __forceinline__ bool is_nan(float v) {
+    uint32_t u = __float_as_uint(v);
+    asm("" : "+v"(u));
+    return (u & 0x7fffffffu) > 0x7f800000u;
 }
 
 constexpr int F32P_WAVES = 4;
@@ -173,19 +183,29 @@ __global__ void __launch_bounds__(64 * F32P_WAVES) attention_f32p_kernel(const T
         mx = halves_max(mx);
         if (__ballot(mx > m_run + rescale) != 0) {
             const float m_new = fmaxf(m_run, mx);
-            const float f = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m_run - m_new) * scale);
+            // (Equal: both minus infinity, or infinite by a score past F32.)
+            const float f = __builtin_amdgcn_exp2f(m_run == m_new ? 0.0f : (m_run - m_new) * scale);
 #pragma unroll
             for (int t = 0; t < NO; ++t) o[t] *= f;
             lsum *= f;
             m_run = m_new;
         }
         const float m = m_run == -INFINITY ? 0.0f : m_run;
-        float pr[16];
+        float pr[16], bsum = 0.0f;
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             pr[i] = __builtin_amdgcn_exp2f(fmaf(sc[i] - m, scale, BIAS));
-            lsum += pr[i];
+            bsum += pr[i];
         }
+        if (__ballot(is_nan(bsum)) != 0) {   // uniform
+            bsum = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                pr[i] = is_nan(pr[i]) ? 0.0f : pr[i];
+                bsum += pr[i];
+            }
+        }
+        lsum += bsum;
         if constexpr (F32) {
 #pragma unroll
             for (int i = 0; i < 16; ++i)
